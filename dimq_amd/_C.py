@@ -831,7 +831,7 @@ def _qat_ws(n, K, device):
 
 
 def softmin_loss_forward_impl(w, centers, tau, mean):
-    """(loss fp32 scalar, aux [n, 2] fp32: (dmin_i, log s_i) for the backward)."""
+    """(loss fp32 scalar, aux [n, 2] fp32: (dmin_i, 1 / s_i) for the backward)."""
     wc, c = _qat_inputs(w, centers)
     n = wc.numel()
     aux = torch.empty((n, 2), dtype=torch.float32, device=wc.device)

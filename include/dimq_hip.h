@@ -440,7 +440,7 @@ int dimq_layer_norm_ex(const void* x, int x_dtype, int64_t rows, int64_t dim, in
  * device), as the reference; d_ij = (w_i - c_j)^2, p_ij = softmax_j(-d_ij/tau).
  * Sums over elements go through per-work-group partials in the caller's
  * workspace (dimq_qat_workspace_bytes) and a fixed-order final pass.
- * aux: 2 floats per element, (min_j d_ij, log sum_j exp(-(d_ij - min d)/tau)),
+ * aux: 2 floats per element, (min_j d_ij, 1 / sum_j exp(-(d_ij - min d)/tau)),
  * written by a forward and read by its backward.
  * ------------------------------------------------------------------------- */
 int64_t dimq_qat_workspace_bytes(int64_t n, int64_t n_centers);

@@ -157,3 +157,27 @@ def test_qat_deterministic_and_errors(gpu):
         qat.dimq_softmin_loss(wd, cd[:0], 1.0)
     with pytest.raises(RuntimeError, match="256"):
         qat.dimq_softmin_loss(wd, torch.zeros(300, device=gpu), 1.0)
+
+
+@pytest.mark.parametrize("n,K", [(1023, 3), (1025, 5), (4096, 9), (3000, 17), (5001, 33), (2_200_003, 4)])
+@pytest.mark.parametrize("tau", [1e-1, 1e-4])
+def test_qat_centre_counts_and_chunk_edges(gpu, n, K, tau):
+    """The register instances (4, 8, 16 centres) at counts below their size, the LDS instance at centre tiles that
+    end early, element counts next to a chunk's edge, and more chunks than work-groups (2,200,003 weights); both
+    functions and the separation loss in one backward."""
+    from dimq_amd import qat
+    announce(f"qat edges n={n} K={K} tau={tau}")
+    w, c = _case(n, K, 5 * n + K)
+    up = torch.randn(n, generator=_gen(n))
+    wd, cd = w.to(gpu).requires_grad_(), c.to(gpu).requires_grad_()
+    y, loss, sep = qat.soft_dequantize_weight(wd, cd, tau), qat.dimq_softmin_loss(wd, cd, tau), qat.separation_loss(wd, cd)
+    gw, gc = torch.autograd.grad((y, loss, sep), (wd, cd), (up.to(gpu), torch.tensor(0.5, device=gpu),
+                                                            torch.tensor(2.0, device=gpu)))
+    wo, co = w.clone().requires_grad_(), c.clone().requires_grad_()
+    yo, lo, so = oqat.soft_dequantize(wo, co, tau), oqat.softmin_loss(wo, co, tau), oqat.separation_loss(w, co)
+    hw, hc = torch.autograd.grad((yo, lo, so), (wo, co), (up.double(), torch.tensor(0.5).double(),
+                                                          torch.tensor(2.0).double()))
+    # the bars of the tests above: 1e-5 of the largest value, 2e-4 for the gradients
+    assert _rel(y.detach(), yo.detach()) <= 1e-5
+    assert _rel(loss.detach(), lo.detach()) <= 2e-5 and _rel(sep.detach(), so.detach()) <= 2e-5
+    assert _rel(gw, hw) <= 2e-4 and _rel(gc, hc) <= 2e-4
