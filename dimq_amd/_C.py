@@ -21,6 +21,8 @@ pointers plus the current HIP stream to the ``extern "C"`` entry point.
 from __future__ import annotations
 
 import ctypes
+from contextlib import nullcontext
+from functools import lru_cache
 from pathlib import Path
 
 import torch  # must be imported first: the HIP runtime comes from torch's libamdhip64
@@ -58,11 +60,13 @@ _SIGS = {
     "dimq_conv2d_lut": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _int, _i64, _dbl, _i64, _vp, _int,
                                _i64] + [_i64] * 11 + [_vp, _vp]),
     "dimq_linear_lut_workspace_bytes": (_i64, [_i64, _i64, _int]),
+    "dimq_linear_lut_full_workspace_bytes": (_i64, [_int, _i64, _i64, _i64, _int]),
     "dimq_linear_lut_ws": (_int, [_vp, _int, _i64, _vp, _i64, _vp, _int, _i64, _dbl, _i64, _vp, _int, _i64, _i64,
                                   _i64, _vp, _vp, _i64, _vp]),
     "dimq_linear_lut_noalloc": (_int, [_vp, _int, _i64, _vp, _i64, _vp, _int, _i64, _dbl, _i64, _vp, _int, _i64,
                                        _i64, _i64, _vp, _vp]),
     "dimq_conv2d_lut_workspace_bytes": (_i64, [_i64] * 9 + [_int]),
+    "dimq_conv2d_lut_full_workspace_bytes": (_i64, [_int] + [_i64] * 15 + [_int]),
     "dimq_conv2d_lut_ws": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _int, _i64, _dbl, _i64, _vp,
                                   _int, _i64] + [_i64] * 11 + [_vp, _vp, _i64, _vp]),
     "dimq_quantize_activation_f16": (_int, [_vp, _int, _i64, _dbl, _i64, _vp, _vp]),
@@ -86,6 +90,7 @@ _SIGS = {
     "dimq_linear_codebook_ex": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _int, _vp, _int, _i64, _i64, _vp, _int,
                                        _i64, _vp, _int, _vp, _int, _int, _int, _vp]),
     "dimq_linear_codebook_workspace_bytes": (_i64, [_i64, _i64, _i64, _int, _int]),
+    "dimq_linear_codebook_full_workspace_bytes": (_i64, [_i64, _i64, _i64, _int, _int]),
     "dimq_linear_codebook_ex_ws": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _int, _vp, _int, _i64, _i64, _vp, _int,
                                           _i64, _vp, _int, _vp, _int, _int, _int, _vp, _i64, _vp]),
     "dimq_codebook_predecode_bytes": (_i64, [_i64, _i64, _int]),
@@ -105,6 +110,11 @@ _SIGS = {
     "dimq_conv2d_codebook_ex": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64, _vp, _i64, _int, _vp, _i64, _vp,
                                        _int, _i64, _i64, _vp, _int] + [_i64] * 10 +
                                 [_vp, _int, _int, _vp, _int, _int, _int, _vp]),
+    "dimq_conv2d_codebook_workspace_bytes": (_i64, [_int, _int] + [_i64] * 4 + [_int, _int, _int] + [_i64] * 12 +
+                                             [_int] * 5),
+    "dimq_conv2d_codebook_ex_ws": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64, _vp, _i64, _int, _vp, _i64, _vp,
+                                          _int, _i64, _i64, _vp, _int] + [_i64] * 10 +
+                                   [_vp, _int, _int, _vp, _int, _int, _int, _vp, _i64, _vp]),
     "dimq_qat_workspace_bytes": (_i64, [_i64, _i64]),
     "dimq_softmin_loss_forward": (_int, [_vp, _int, _i64, _vp, _i64, _dbl, _int, _vp, _vp, _vp, _i64, _vp]),
     "dimq_softmin_loss_backward": (_int, [_vp, _int, _i64, _vp, _i64, _dbl, _int, _vp, _vp, _vp, _int, _vp, _vp, _i64,
@@ -137,6 +147,20 @@ def _ptr(t: torch.Tensor | None):
 
 def _stream(device: torch.device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+_SAME_DEVICE = nullcontext()
+
+
+def _on(device: torch.device):
+    """Context with `device` current (nothing to do where it already is)."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+@lru_cache(maxsize=1024)
+def _conv_workspace_bytes(*sizes) -> int:
+    """dimq_conv2d_codebook_workspace_bytes: a function of the call's sizes, dtypes and options alone."""
+    return lib.dimq_conv2d_codebook_workspace_bytes(*sizes)
 
 
 def _dtype(t: torch.Tensor) -> int:
@@ -250,8 +274,9 @@ def linear_lut_impl(x, packed_w, codebook, act_scale, act_zp, bias, out_features
     b, bp, bdt, bn = _bias_args(bias, out_features, "out_features")
     M = xc.numel() // in_features
     y = torch.empty((M, out_features), dtype=torch.float32, device=xc.device)
-    ws = _workspace(lib.dimq_linear_lut_workspace_bytes(M, in_features, _dtype(cb)), xc.device)
-    with torch.cuda.device(xc.device):
+    ws = _workspace(lib.dimq_linear_lut_full_workspace_bytes(_dtype(xc), M, out_features, in_features, _dtype(cb)),
+                    xc.device)
+    with _on(xc.device):
         _check(lib.dimq_linear_lut_ws(_ptr(xc), _dtype(xc), M, _ptr(pw), pw.numel(), _ptr(cb), _dtype(cb), cb.numel(),
                                       float(act_scale), int(act_zp), bp, bdt, bn, out_features, in_features, _ptr(y),
                                       _ptr(ws), 0 if ws is None else ws.numel(), _stream(xc.device)))
@@ -281,9 +306,10 @@ def conv2d_lut_impl(x, packed_w, codebook, act_scale, act_zp, bias, out_channels
     y = torch.empty((B, out_channels, max(oh, 0), max(ow, 0)), dtype=torch.float32, device=xc.device)
     ws = None
     if y.numel() > 0:
-        ws = _workspace(lib.dimq_conv2d_lut_workspace_bytes(B, C, H, W, out_channels, in_channels_per_group, kernel_h,
-                                                            kernel_w, groups, _dtype(cb)), xc.device)
-    with torch.cuda.device(xc.device):
+        ws = _workspace(lib.dimq_conv2d_lut_full_workspace_bytes(
+            _dtype(xc), B, C, H, W, out_channels, in_channels_per_group, kernel_h, kernel_w, stride_h, stride_w, pad_h,
+            pad_w, dilation_h, dilation_w, groups, _dtype(cb)), xc.device)
+    with _on(xc.device):
         _check(lib.dimq_conv2d_lut_ws(_ptr(xc), _dtype(xc), B, C, H, W, _ptr(pw), pw.numel(), _ptr(cb), _dtype(cb),
                                       cb.numel(), float(act_scale), int(act_zp), bp, bdt, bn, out_channels,
                                       in_channels_per_group, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
@@ -397,9 +423,9 @@ def linear_codebook_impl(x, packed_w, codebook, bits, bias, out_features, in_fea
         raise RuntimeError(f"residual shape {tuple(residual.shape)} must equal the output shape "
                            f"{(*x.shape[:-1], out_features)}")
     r, rp, rdt = _residual_args(None if residual is None else residual.reshape(M, out_features), y)
-    ws = _workspace(lib.dimq_linear_codebook_workspace_bytes(M, in_features, out_features, int(bits), _dtype(xc)),
+    ws = _workspace(lib.dimq_linear_codebook_full_workspace_bytes(M, in_features, out_features, int(bits), _dtype(xc)),
                     xc.device)
-    with torch.cuda.device(xc.device):
+    with _on(xc.device):
         if decoded is None:
             _check(lib.dimq_linear_codebook_ex_ws(_ptr(xc), _dtype(xc), M, in_features, _ptr(pw), pw.numel(),
                                                   int(bits), _ptr(cb), _dtype(cb), rows, size, bp, bdt, out_features,
@@ -677,12 +703,17 @@ def conv2d_codebook_impl(x, packed_w, codebook, bits, bias, out_channels, in_cha
     else:
         prep_ptr, prep_words = None, 0
     r, rp, rdt = _residual_args(residual, y, mf)
-    with torch.cuda.device(xc.device):
-        _check(lib.dimq_conv2d_codebook_ex(_ptr(xc), _dtype(xc), layout, B, C, H, W, _ptr(pw), pw.numel(), int(bits),
-                                           prep_ptr, prep_words, _ptr(cb), _dtype(cb), rows, size, bp, bdt,
-                                           out_channels, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
-                                           dilation_h, dilation_w, groups, _ptr(y), _dtype(y), layout, rp, rdt,
-                                           int(activation), int(variant), _stream(xc.device)))
+    ws = _workspace(_conv_workspace_bytes(
+        _dtype(xc), layout, B, C, H, W, int(bits), int(prep_words > 0), _dtype(cb), rows, size, out_channels, kernel_h,
+        kernel_w, stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, groups, _dtype(y), layout,
+        int(r is not None), int(activation), int(variant)), xc.device)
+    with _on(xc.device):
+        _check(lib.dimq_conv2d_codebook_ex_ws(_ptr(xc), _dtype(xc), layout, B, C, H, W, _ptr(pw), pw.numel(),
+                                              int(bits), prep_ptr, prep_words, _ptr(cb), _dtype(cb), rows, size, bp,
+                                              bdt, out_channels, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
+                                              dilation_h, dilation_w, groups, _ptr(y), _dtype(y), layout, rp, rdt,
+                                              int(activation), int(variant), _ptr(ws),
+                                              0 if ws is None else ws.numel(), _stream(xc.device)))
     return y
 
 

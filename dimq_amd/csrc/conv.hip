@@ -2,6 +2,7 @@
 // from csrc/dimq_conv2d_lut.cu:105-134) and launch of the implicit-GEMM
 // kernels (im2col gathered on the fly, never materialised).
 #include "gemm_big.h"
+#include "gemm_gen.h"
 
 namespace dimq {
 namespace {
@@ -156,6 +157,11 @@ int gemm_conv_tile(int64_t M, int64_t N, int64_t K) {
   return t128 >= device_cus() ? 0 : 1;
 }
 
+// The conv's arguments as the general pre-laid path's plan reads them (no pointers).
+GemmArgs shape_args(const ConvShape& s, int x_layout, int y_layout, int cb_dt) {
+  return conv_args(s, nullptr, x_layout, nullptr, nullptr, cb_dt, 1, 1, nullptr, DIMQ_F32, nullptr, DIMQ_F32, y_layout);
+}
+
 ConvShape make_shape(int64_t B, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t ICg, int64_t KH, int64_t KW,
                      int64_t sh, int64_t sw, int64_t ph, int64_t pw, int64_t dh, int64_t dw, int64_t groups) {
   ConvShape s{B, C, H, W, OC, ICg, KH, KW, sh, sw, ph, pw, dh, dw, groups, 0, 0};
@@ -197,6 +203,30 @@ extern "C" int64_t dimq_conv2d_lut_workspace_bytes(int64_t B, int64_t C, int64_t
   const int64_t hw = (groups == 1 && in_channels_per_group == C)
                          ? halo_part_words(out_channels, C, kernel_h, kernel_w, 4) : 0;
   return lut_act_bytes(B, C, H, W) + hw * 4;
+}
+
+// dimq_conv2d_lut_workspace_bytes, or what the general pre-laid path needs
+// where that path runs: any shape the LDS-halo kernels do not, any codebook
+// dtype.
+static bool lut_halo(const ConvShape& s, int cb_dtype) {
+  return cb_dtype == DIMQ_F16 && s.groups == 1 && halo_part_words(s.OC, s.C, s.KH, s.KW, 4) > 0 &&
+         halo_eligible(s.C, s.KH, s.KW, s.sh, s.sw, s.dh, s.dw, s.groups, s.OH, s.OW, 4, DIMQ_F16, kEpiNone, DIMQ_NCHW);
+}
+
+extern "C" int64_t dimq_conv2d_lut_full_workspace_bytes(int x_dtype, int64_t B, int64_t C, int64_t H, int64_t W,
+                                                        int64_t out_channels, int64_t in_channels_per_group,
+                                                        int64_t kernel_h, int64_t kernel_w, int64_t stride_h,
+                                                        int64_t stride_w, int64_t pad_h, int64_t pad_w,
+                                                        int64_t dilation_h, int64_t dilation_w, int64_t groups,
+                                                        int cb_dtype) {
+  const int64_t small = dimq_conv2d_lut_workspace_bytes(B, C, H, W, out_channels, in_channels_per_group, kernel_h,
+                                                        kernel_w, groups, cb_dtype);
+  if (groups <= 0 || out_channels <= 0 || kernel_h <= 0 || kernel_w <= 0 || stride_h <= 0 || stride_w <= 0) return small;
+  const ConvShape s = make_shape(B, C, H, W, out_channels, in_channels_per_group, kernel_h, kernel_w, stride_h,
+                                 stride_w, pad_h, pad_w, dilation_h, dilation_w, groups);
+  if (s.OH <= 0 || s.OW <= 0 || lut_halo(s, cb_dtype)) return small;
+  const GenPlan g = gen_plan(shape_args(s, DIMQ_NCHW, DIMQ_NCHW, cb_dtype), 4, x_dtype, true, true);
+  return g.ok && g.bytes > small ? g.bytes : small;
 }
 
 extern "C" int dimq_conv2d_lut(const void* x, int x_dtype, int64_t B, int64_t C, int64_t H, int64_t W,
@@ -241,6 +271,14 @@ extern "C" int dimq_conv2d_lut_ws(const void* x, int x_dtype, int64_t B, int64_t
   DIMQ_CHECK(workspace_bytes >= 0, "workspace_bytes must be non-negative");
   if (s.B * s.OC * s.OH * s.OW == 0) return DIMQ_OK;
   const hipStream_t st = as_stream(stream);
+  if (workspace != nullptr && aligned(workspace, 256) && !lut_halo(s, cb_dtype)) {
+    GemmArgs p = conv_args(s, x, DIMQ_NCHW, packed_w, codebook, cb_dtype, 1, 16, bias, bias_dtype, y, DIMQ_F32,
+                           DIMQ_NCHW);
+    p.acc_scale = p.act_scale = static_cast<float>(act_scale);
+    p.act_zp = static_cast<int>(act_zp);
+    const GenPlan g = gen_plan(p, 4, x_dtype, true, true);
+    if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, 4, x_dtype, workspace, st);
+  }
   const int64_t need = dimq_conv2d_lut_workspace_bytes(s.B, s.C, s.H, s.W, s.OC, s.ICg, s.KH, s.KW, s.groups,
                                                        cb_dtype);
   if (workspace != nullptr && need > 0 && workspace_bytes >= need && aligned(workspace, 16)) {
@@ -413,6 +451,77 @@ extern "C" int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout,
                                        int64_t dilation_h, int64_t dilation_w, int64_t groups, void* y, int y_dtype,
                                        int y_layout, const void* residual, int residual_dtype, int activation,
                                        int variant, void* stream) {
+  return dimq_conv2d_codebook_ex_ws(x, x_dtype, x_layout, B, C, H, W, packed_w, packed_numel, bits, prepared_w,
+                                    prepared_words, codebook, cb_dtype, cb_rows, cb_size, bias, bias_dtype,
+                                    out_channels, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w, dilation_h,
+                                    dilation_w, groups, y, y_dtype, y_layout, residual, residual_dtype, activation,
+                                    variant, nullptr, 0, stream);
+}
+
+// The kernel family of a weight-only conv with epilogue `mode`.  x16: x is
+// 16-byte aligned, yw16: y and the prepared weights are; stem: the stem
+// kernel's own test holds.
+enum ConvPath { kConvGemm, kConvHalo, kConvStem, kConvGeneral };
+
+static ConvPath conv_path(const ConvShape& s, int x_dtype, int x_layout, int y_dtype, int y_layout, int bits,
+                          bool prepared, int mode, int variant, bool x16, bool yw16, bool stem) {
+  (void)y_dtype;
+  const int64_t hw = prepared ? halo_part_words(s.OC, s.C, s.KH, s.KW, bits) : 0;
+  const int64_t gw = prepared ? gemm_part_words(s.OC, s.C, s.KH, s.KW, bits) : 0;
+  const bool gemm_ok = gw > 0 && variant != DIMQ_VARIANT_SMALL_M && s.groups == 1 && x_layout == DIMQ_NHWC &&
+                       (mode == kEpiNone || mode == kEpiRelu || mode == kEpiRes || mode == kEpiResRelu) &&
+                       y_layout == DIMQ_NHWC && (x_dtype == DIMQ_F16 || x_dtype == DIMQ_BF16) && x16 && yw16;
+  const bool halo_ok = hw > 0 && variant != DIMQ_VARIANT_SMALL_M && x16 &&
+                       halo_eligible(s.C, s.KH, s.KW, s.sh, s.sw, s.dh, s.dw, s.groups, s.OH, s.OW, bits, x_dtype,
+                                     mode, y_layout);
+  // DIMQ_VARIANT_MFMA forces the implicit-GEMM tiles over the LDS-halo kernel
+  // (A/B runs of the choice prefer_gemm_conv makes)
+  if (gemm_ok && (!halo_ok || variant == DIMQ_VARIANT_MFMA || prefer_gemm_conv(s.C, s.KH, s.KW, s.sh))) return kConvGemm;
+  if (halo_ok) return kConvHalo;
+  if (variant != DIMQ_VARIANT_SMALL_M && stem) return kConvStem;
+  return kConvGeneral;
+}
+
+// Workspace with which dimq_conv2d_codebook_ex_ws runs the general pre-laid
+// path on a call whose pointers are 16-byte aligned; 0 when another kernel
+// takes the shape.
+extern "C" int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H,
+                                                        int64_t W, int bits, int prepared, int cb_dtype,
+                                                        int64_t cb_rows, int64_t cb_size, int64_t out_channels, int64_t kernel_h, int64_t kernel_w,
+                                                        int64_t stride_h, int64_t stride_w, int64_t pad_h,
+                                                        int64_t pad_w, int64_t dilation_h, int64_t dilation_w,
+                                                        int64_t groups, int y_dtype, int y_layout, int residual,
+                                                        int activation, int variant) {
+  if (B <= 0 || C <= 0 || H <= 0 || W <= 0 || out_channels <= 0 || kernel_h <= 0 || kernel_w <= 0 || stride_h <= 0 ||
+      stride_w <= 0 || dilation_h <= 0 || dilation_w <= 0 || pad_h < 0 || pad_w < 0 || groups <= 0 || C % groups != 0 ||
+      out_channels % groups != 0 || variant == DIMQ_VARIANT_SMALL_M)
+    return 0;
+  const ConvShape s = make_shape(B, C, H, W, out_channels, C / groups, kernel_h, kernel_w, stride_h, stride_w, pad_h,
+                                 pad_w, dilation_h, dilation_w, groups);
+  if (s.OH <= 0 || s.OW <= 0) return 0;
+  const int mode = (residual ? kEpiRes : 0) | activation;
+  // 16-byte aligned pointers of the stem kernel's own test
+  const void* al = reinterpret_cast<const void*>(static_cast<uintptr_t>(256));
+  const bool stem = stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits,
+                                  x_dtype, y_dtype, al, al, mode, static_cast<const uint8_t*>(al),
+                                  (s.OC * s.ICg * s.KH * s.KW * bits + 7) / 8, al, cb_dtype, cb_rows, cb_size);
+  if (conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared != 0, mode, variant, true, true, stem) !=
+      kConvGeneral)
+    return 0;
+  const GenPlan g = gen_plan(shape_args(s, x_layout, y_layout, DIMQ_F32), bits, x_dtype, false, true);
+  return g.ok ? g.bytes : 0;
+}
+
+extern "C" int dimq_conv2d_codebook_ex_ws(const void* x, int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H,
+                                          int64_t W, const uint8_t* packed_w, int64_t packed_numel, int bits,
+                                          const uint32_t* prepared_w, int64_t prepared_words, const void* codebook,
+                                          int cb_dtype, int64_t cb_rows, int64_t cb_size, const void* bias,
+                                          int bias_dtype, int64_t out_channels, int64_t kernel_h, int64_t kernel_w,
+                                          int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
+                                          int64_t dilation_h, int64_t dilation_w, int64_t groups, void* y, int y_dtype,
+                                          int y_layout, const void* residual, int residual_dtype, int activation,
+                                          int variant, void* workspace, int64_t workspace_bytes, void* stream) {
+  DIMQ_CHECK(workspace_bytes >= 0, "workspace_bytes must be non-negative");
   if (!(bits == 2 || bits == 3 || bits == 4 || bits == 8))
     return set_error(DIMQ_ERR_UNSUPPORTED, "bits must be one of 2, 3, 4, 8 (got %d)", bits);
   DIMQ_CHECK(x_dtype == DIMQ_F32 || x_dtype == DIMQ_F16 || x_dtype == DIMQ_BF16,
@@ -442,16 +551,12 @@ extern "C" int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout,
   const int64_t gw = prepared_w ? gemm_part_words(s.OC, s.C, s.KH, s.KW, bits) : 0;
   if (prepared_w != nullptr) DIMQ_CHECK(prepared_words >= hw + gw, "prepared weight buffer is too small");
   const int mode = epi_mode(epi);
-  const bool gemm_ok = gw > 0 && variant != DIMQ_VARIANT_SMALL_M && s.groups == 1 && x_layout == DIMQ_NHWC &&
-                       (mode == kEpiNone || mode == kEpiRelu || mode == kEpiRes || mode == kEpiResRelu) &&
-                       y_layout == DIMQ_NHWC && (x_dtype == DIMQ_F16 || x_dtype == DIMQ_BF16) && aligned(x, 16) &&
-                       aligned(y, 16) && aligned(prepared_w + hw, 16);
-  const bool halo_ok = hw > 0 && variant != DIMQ_VARIANT_SMALL_M && aligned(x, 16) &&
-                       halo_eligible(s.C, s.KH, s.KW, s.sh, s.sw, s.dh, s.dw, s.groups, s.OH, s.OW, bits, x_dtype,
-                                     epi_mode(epi), y_layout);
-  // DIMQ_VARIANT_MFMA forces the implicit-GEMM tiles over the LDS-halo kernel
-  // (A/B runs of the choice prefer_gemm_conv makes)
-  if (gemm_ok && (!halo_ok || variant == DIMQ_VARIANT_MFMA || prefer_gemm_conv(s.C, s.KH, s.KW, s.sh))) {
+  const bool stem = stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits,
+                                  x_dtype, y_dtype, x, y, mode, packed_w, packed_numel, codebook, cb_dtype, cb_rows,
+                                  cb_size);
+  const ConvPath path = conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared_w != nullptr, mode, variant,
+                                  aligned(x, 16), aligned(y, 16) && aligned(prepared_w + hw, 16), stem);
+  if (path == kConvGemm) {
     GemmArgs p = conv_args(s, x, x_layout, reinterpret_cast<const uint8_t*>(prepared_w + hw), codebook, cb_dtype,
                            cb_rows, cb_size, bias, bias_dtype, y, y_dtype, y_layout);
     p.ldy = s.OC;
@@ -463,14 +568,12 @@ extern "C" int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout,
       default: return launch_big_conv_b4(p, x_dtype, tile, as_stream(stream));
     }
   }
-  if (halo_ok) {
+  if (path == kConvHalo) {
     return launch_conv_halo(x, x_dtype, x_layout, s.B, s.C, s.H, s.W, prepared_w, bits, codebook, cb_dtype, cb_rows,
                             cb_size, bias, bias_dtype, s.OC, s.KH, s.KW, s.sh, s.ph, s.pw, s.OH, s.OW, y, y_dtype,
                             y_layout, epi, as_stream(stream));
   }
-  if (variant != DIMQ_VARIANT_SMALL_M &&
-      stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits, x_dtype, y_dtype, x, y,
-                    epi_mode(epi), packed_w, packed_numel, codebook, cb_dtype, cb_rows, cb_size)) {
+  if (path == kConvStem) {
     return launch_conv_stem(x, x_dtype, x_layout, s.B, s.C, s.H, s.W, packed_w, packed_numel, bits, codebook,
                             cb_dtype, cb_rows, cb_size, bias, bias_dtype, s.OC, s.KH, s.KW, s.ph, s.pw, s.OH, s.OW,
                             y, y_dtype, y_layout, epi, as_stream(stream));
@@ -478,6 +581,10 @@ extern "C" int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout,
   GemmArgs p = conv_args(s, x, x_layout, packed_w, codebook, cb_dtype, cb_rows, cb_size, bias, bias_dtype, y,
                          y_dtype, y_layout);
   p.epi = epi;
+  if (workspace != nullptr && aligned(workspace, 256) && variant != DIMQ_VARIANT_SMALL_M) {
+    const GenPlan g = gen_plan(p, bits, x_dtype, false, aligned(x, 16));
+    if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, bits, x_dtype, workspace, as_stream(stream));
+  }
   int tile = gemm_pick_tile(p.M, p.N, variant);
   if (tile == kTileGemv) tile = kTile16x16;  // the GEMV kernel has no im2col/group support
   return gemm_dispatch(p, bits, x_dtype, false, tile, as_stream(stream));

@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "gemm_big.h"
+#include "gemm_gen.h"
 #include "gemm_kernel.h"
 #include "gemv_fast.h"
 
@@ -47,6 +48,20 @@ int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
   // the CUs better (M 1000: 17 vs 30 us).
   if (p.M >= 2048 && x_dtype != DIMQ_F32) return 10;  // fp32 activations spill its registers
   return p.K >= 2048 ? 2 : 7;
+}
+
+// Whether the general pre-laid path (gemm_gen.hip) takes a Linear that no path
+// with a workspace of its own does: every shape beyond the decode shapes that
+// the large tiles' k steps or codebooks do not fit.  At 16 < M <= 64 with
+// K % 128 == 0 the register-codebook tiles decode each weight once or twice
+// only, and win while K is short (M 17, K 384, N 3,072: 11.7 against 12.2 us;
+// M 32, K 3,072, N 768: 30.4 against 16.8).
+// And while the weights are few: laying out 16.8 M of them takes 25 us (M 20,
+// K = N = 4,096: 38.8 against 43.1).
+bool gen_wants_linear(int64_t M, int64_t K, int64_t N, int bits) {
+  if (M <= 16) return false;
+  if (bits == 8 || K % 64 != 0) return true;
+  return M <= 64 && (K % 128 != 0 || (K >= 1024 && N * K <= (8ll << 20)));
 }
 
 int gemm_pick_tile(int64_t M, int64_t N, int variant) {
@@ -128,6 +143,11 @@ int linear_codebook_impl(const void* x, int x_dtype, int64_t M, int64_t K, int64
     if (rc >= 0) return rc;
   }
   const int big = gemm_big_tile(p, bits, x_dtype, variant);
+  if (big < 0 && M > 16 && (M > 64 || gen_wants_linear(M, K, N, bits)) && workspace != nullptr &&
+      aligned(workspace, 256) && variant != DIMQ_VARIANT_SMALL_M) {
+    const GenPlan g = gen_plan(p, bits, x_dtype, false, aligned(x, 16));
+    if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, bits, x_dtype, workspace, s);
+  }
   if (big >= 0) {
     switch (bits) {
       case 2: return launch_big_b2(p, x_dtype, big, s);
@@ -203,6 +223,26 @@ extern "C" int64_t dimq_linear_codebook_workspace_bytes(int64_t M, int64_t K, in
   return (gemv_partial_bytes(p, pl) + 255) / 256 * 256;
 }
 
+// The arguments of a Linear as the general pre-laid path's plan reads them (no pointers).
+static GemmArgs linear_shape_args(int64_t M, int64_t K, int64_t N, int cb_dtype) {
+  GemmArgs p{};
+  p.M = M;
+  p.K = p.ldx = K;
+  p.N = p.ldy = N;
+  p.cb_dt = cb_dtype;
+  p.groups = 1;
+  return p;
+}
+
+// dimq_linear_codebook_workspace_bytes, or what the general pre-laid path
+// needs where no other path with a workspace takes the shape.
+extern "C" int64_t dimq_linear_codebook_full_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype) {
+  const int64_t own = dimq_linear_codebook_workspace_bytes(M, K, N, bits, x_dtype);
+  if (own > 0 || M <= 0 || K <= 0 || N <= 0 || !gen_wants_linear(M, K, N, bits)) return own;
+  const GenPlan g = gen_plan(linear_shape_args(M, K, N, DIMQ_F32), bits, x_dtype, false, true);
+  return g.ok ? g.bytes : 0;
+}
+
 extern "C" int dimq_linear_codebook_ex_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint8_t* packed_w,
                                           int64_t packed_numel, int bits, const void* codebook, int cb_dtype,
                                           int64_t cb_rows, int64_t cb_size, const void* bias, int bias_dtype,
@@ -210,10 +250,9 @@ extern "C" int dimq_linear_codebook_ex_ws(const void* x, int x_dtype, int64_t M,
                                           int activation, int variant, void* workspace, int64_t workspace_bytes,
                                           void* stream) {
   DIMQ_CHECK(workspace_bytes >= 0, "workspace_bytes must be non-negative");
-  const bool decode = (M >= 1 && M <= 16) || predecoded_ws_bytes(M, K, N, bits, x_dtype) > 0;
   return linear_codebook_checked(x, x_dtype, M, K, packed_w, packed_numel, bits, codebook, cb_dtype, cb_rows, cb_size,
                                  bias, bias_dtype, N, y, y_dtype, residual, residual_dtype, activation, variant,
-                                 stream, decode ? workspace : nullptr, decode ? workspace_bytes : 0);
+                                 stream, workspace, workspace_bytes);
 }
 
 extern "C" int64_t dimq_codebook_predecode_bytes(int64_t out_features, int64_t in_features, int bits) {
@@ -248,10 +287,9 @@ extern "C" int dimq_linear_codebook_predecoded(const void* x, int x_dtype, int64
                                                void* stream) {
   DIMQ_CHECK(workspace_bytes >= 0, "workspace_bytes must be non-negative");
   DIMQ_CHECK(decoded == nullptr || aligned(decoded, 256), "decoded must be 256-byte aligned");
-  const bool decode = (M >= 1 && M <= 16) || predecoded_ws_bytes(M, K, N, bits, x_dtype) > 0;
   return linear_codebook_checked(x, x_dtype, M, K, packed_w, packed_numel, bits, codebook, cb_dtype, cb_rows, cb_size,
                                  bias, bias_dtype, N, y, y_dtype, residual, residual_dtype, activation, variant,
-                                 stream, decode ? workspace : nullptr, decode ? workspace_bytes : 0, decoded);
+                                 stream, workspace, workspace_bytes, decoded);
 }
 
 extern "C" int64_t dimq_linear_codebook_act_workspace_bytes(int64_t M, int64_t K) {
@@ -345,6 +383,21 @@ extern "C" int64_t dimq_linear_lut_workspace_bytes(int64_t M, int64_t in_feature
   return (M * in_features * 2 + 255) / 256 * 256;
 }
 
+// dimq_linear_lut_workspace_bytes, or what the general pre-laid path needs
+// where that path runs: codebooks that are not fp16, and in_features off the
+// fast tiles' k steps.
+static bool lut_wants_gen(int64_t M, int64_t in_features, int64_t out_features, int cb_dtype) {
+  return cb_dtype != DIMQ_F16 || gen_wants_linear(M, in_features, out_features, 4);
+}
+
+extern "C" int64_t dimq_linear_lut_full_workspace_bytes(int x_dtype, int64_t M, int64_t out_features,
+                                                        int64_t in_features, int cb_dtype) {
+  const int64_t small = dimq_linear_lut_workspace_bytes(M, in_features, cb_dtype);
+  if (M <= 0 || out_features <= 0 || in_features <= 0 || !lut_wants_gen(M, in_features, out_features, cb_dtype)) return small;
+  const GenPlan g = gen_plan(linear_shape_args(M, in_features, out_features, cb_dtype), 4, x_dtype, true, true);
+  return g.ok && g.bytes > small ? g.bytes : small;
+}
+
 extern "C" int dimq_linear_lut(const void* x, int x_dtype, int64_t M, const uint8_t* packed_w, int64_t packed_numel,
                                const void* codebook, int cb_dtype, int64_t cb_numel, double act_scale,
                                int64_t act_zp, const void* bias, int bias_dtype, int64_t bias_numel,
@@ -388,6 +441,22 @@ extern "C" int dimq_linear_lut_ws(const void* x, int x_dtype, int64_t M, const u
   if (rc0 != DIMQ_OK) return rc0;
   DIMQ_CHECK(workspace_bytes >= 0, "workspace_bytes must be non-negative");
   if (M == 0) return DIMQ_OK;
+  if (workspace != nullptr && aligned(workspace, 256) && lut_wants_gen(M, in_features, out_features, cb_dtype)) {
+    GemmArgs p = linear_shape_args(M, in_features, out_features, cb_dtype);
+    p.x = x;
+    p.w = packed_w;
+    p.cb = codebook;
+    p.cb_rows = 1;
+    p.cb_size = 16;
+    p.bias = bias;
+    p.bias_dt = bias_dtype;
+    p.y = y;
+    p.y_dt = DIMQ_F32;
+    p.acc_scale = p.act_scale = static_cast<float>(act_scale);
+    p.act_zp = static_cast<int>(act_zp);
+    const GenPlan g = gen_plan(p, 4, x_dtype, true, true);
+    if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, 4, x_dtype, workspace, as_stream(stream));
+  }
   const int64_t need = dimq_linear_lut_workspace_bytes(M, in_features, cb_dtype);
   if (workspace != nullptr && need > 0 && workspace_bytes >= need && aligned(workspace, 16)) {
     uint16_t* q = static_cast<uint16_t*>(workspace);

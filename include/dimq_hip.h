@@ -120,6 +120,12 @@ int dimq_conv2d_lut(const void* x, int x_dtype, int64_t B, int64_t C, int64_t H,
  * written on `stream`: calls that share one must be ordered on that stream.
  * *_workspace_bytes returns 0 when no workspace is used for the shape. */
 int64_t dimq_linear_lut_workspace_bytes(int64_t M, int64_t in_features, int cb_dtype);
+/* The same, or for calls the general pre-laid path takes (codebooks that are
+ * not fp16, in_features off the fast tiles' k steps) that path's workspace:
+ * weights and activations laid out as fp16, and fp32 partial outputs where the
+ * k range is split.  A smaller workspace keeps the other kernels. */
+int64_t dimq_linear_lut_full_workspace_bytes(int x_dtype, int64_t M, int64_t out_features, int64_t in_features,
+                                             int cb_dtype);
 int dimq_linear_lut_ws(const void* x, int x_dtype, int64_t M, const uint8_t* packed_w, int64_t packed_numel,
                        const void* codebook, int cb_dtype, int64_t cb_numel, double act_scale, int64_t act_zp,
                        const void* bias, int bias_dtype, int64_t bias_numel, int64_t out_features,
@@ -127,6 +133,13 @@ int dimq_linear_lut_ws(const void* x, int x_dtype, int64_t M, const uint8_t* pac
 int64_t dimq_conv2d_lut_workspace_bytes(int64_t B, int64_t C, int64_t H, int64_t W, int64_t out_channels,
                                         int64_t in_channels_per_group, int64_t kernel_h, int64_t kernel_w,
                                         int64_t groups, int cb_dtype);
+/* The same, or the general pre-laid path's workspace for shapes the LDS-halo
+ * kernels do not run and codebooks that are not fp16. */
+int64_t dimq_conv2d_lut_full_workspace_bytes(int x_dtype, int64_t B, int64_t C, int64_t H, int64_t W,
+                                             int64_t out_channels, int64_t in_channels_per_group, int64_t kernel_h,
+                                             int64_t kernel_w, int64_t stride_h, int64_t stride_w, int64_t pad_h,
+                                             int64_t pad_w, int64_t dilation_h, int64_t dilation_w, int64_t groups,
+                                             int cb_dtype);
 int dimq_conv2d_lut_ws(const void* x, int x_dtype, int64_t B, int64_t C, int64_t H, int64_t W,
                        const uint8_t* packed_w, int64_t packed_numel, const void* codebook, int cb_dtype,
                        int64_t cb_numel, double act_scale, int64_t act_zp, const void* bias, int bias_dtype,
@@ -302,6 +315,9 @@ int dimq_linear_codebook_ex(const void* x, int x_dtype, int64_t M, int64_t K, co
  * workspace.  The workspace is written on `stream`; calls sharing one must
  * be ordered on it. */
 int64_t dimq_linear_codebook_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype);
+/* The same, or for shapes without such a path (8-bit codebooks, in_features
+ * off the k steps, 16 < M <= 64) the general pre-laid path's workspace. */
+int64_t dimq_linear_codebook_full_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype);
 int dimq_linear_codebook_ex_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint8_t* packed_w,
                                int64_t packed_numel, int bits, const void* codebook, int cb_dtype, int64_t cb_rows,
                                int64_t cb_size, const void* bias, int bias_dtype, int64_t N, void* y, int y_dtype,
@@ -414,6 +430,27 @@ int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout, int64_t B,
                             int64_t pad_w, int64_t dilation_h, int64_t dilation_w, int64_t groups, void* y,
                             int y_dtype, int y_layout, const void* residual, int residual_dtype, int activation,
                             int variant, void* stream);
+/* dimq_conv2d_codebook_ex with a workspace (nullable; 256-byte aligned): shapes
+ * that no shape-specific kernel takes (NCHW or fp32 / bf16 input off those
+ * kernels' forms, groups, dilation, 8-bit, odd channel counts) lay weights and
+ * activations out in it as fp16 and run the general pre-laid path, when it
+ * holds dimq_conv2d_codebook_workspace_bytes (0: another kernel takes the
+ * call).  `prepared`, `residual`: whether the call passes one. */
+int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H, int64_t W,
+                                             int bits, int prepared, int cb_dtype, int64_t cb_rows, int64_t cb_size,
+                                             int64_t out_channels, int64_t kernel_h, int64_t kernel_w,
+                                             int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
+                                             int64_t dilation_h, int64_t dilation_w, int64_t groups, int y_dtype,
+                                             int y_layout, int residual, int activation, int variant);
+int dimq_conv2d_codebook_ex_ws(const void* x, int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H, int64_t W,
+                            const uint8_t* packed_w, int64_t packed_numel, int bits, const uint32_t* prepared_w,
+                            int64_t prepared_words, const void* codebook, int cb_dtype, int64_t cb_rows,
+                            int64_t cb_size, const void* bias, int bias_dtype, int64_t out_channels,
+                            int64_t kernel_h, int64_t kernel_w, int64_t stride_h, int64_t stride_w, int64_t pad_h,
+                            int64_t pad_w, int64_t dilation_h, int64_t dilation_w, int64_t groups, void* y,
+                            int y_dtype, int y_layout, const void* residual, int residual_dtype, int activation,
+                            int variant, void* workspace,
+                               int64_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * 3. Support ops of the end-to-end workloads (not DIMQ ops: the reference
