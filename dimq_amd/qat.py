@@ -14,7 +14,8 @@ results, for CUDA (HIP) tensors.
   gradient to ``w``).
 
 ``chunk_size`` is accepted for signature compatibility: the kernels stream the weights and
-need no chunking.  Everything is computed in fp32 from ``w.float()`` and ``centers.float()``;
+need no chunking.  The functions with a backward of their own are autograd nodes of the compiled
+half (``csrc/native.cpp``).  Everything is computed in fp32 from ``w.float()`` and ``centers.float()``;
 the loss values are fp32 scalars on the device.
 """
 
@@ -23,7 +24,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import _C
+from ._C import _native
 
 
 def _tau(tau: float) -> float:
@@ -41,65 +42,21 @@ def hard_quantize_weight(w: Tensor, centers: Tensor, chunk_size: int | None = 26
     return c[idx].to(dtype=w.dtype), idx
 
 
-class _STE(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, w: Tensor, centers: Tensor) -> Tensor:
-        from . import ops
-
-        _, vals = ops.hard_quantize(w.detach(), centers.detach().reshape(-1).float(), False)
-        return vals.reshape(w.shape).to(w.dtype)
-
-    @staticmethod
-    def backward(ctx, grad: Tensor):
-        return grad, None
-
-
 def fake_quant_weight_ste(w: Tensor, centers: Tensor) -> Tensor:
     """The ``hard_ste`` forward of the QAT wrappers (quant/dimq_wrapper.py:78-80): the hard-quantized weight
     forward, the straight-through identity to ``w`` backward."""
-    return _STE.apply(w, centers)
+    return _native.hard_ste(w, centers)
 
 
 def fake_quant_activation_ste(x: Tensor, activation_centers: Tensor) -> Tensor:
     """Activations to their nearest activation centre, straight through backward (quant/dimq_wrapper.py:84-86,
     without the wrapper's running centre update)."""
-    return _STE.apply(x, activation_centers)
-
-
-class _SoftDequant(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, w: Tensor, centers: Tensor, tau: float) -> Tensor:
-        out, aux = _C.soft_dequantize_forward_impl(w, centers, tau)
-        ctx.save_for_backward(w, centers, aux)
-        ctx.tau = tau
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out: Tensor):
-        w, centers, aux = ctx.saved_tensors
-        gw, gc = _C.soft_dequantize_backward_impl(w, centers, ctx.tau, aux, grad_out)
-        return gw, gc.to(centers.dtype).reshape(centers.shape), None
+    return _native.hard_ste(x, activation_centers)
 
 
 def soft_dequantize_weight(w: Tensor, centers: Tensor, tau: float, chunk_size: int | None = 262144) -> Tensor:
     """``softmax(-(w - c)^2 / tau) @ c`` per element, in w's dtype (quant/dimq.py:224-241)."""
-    return _SoftDequant.apply(w, centers, _tau(tau))
-
-
-class _Softmin(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, w: Tensor, centers: Tensor, tau: float, mean: bool) -> Tensor:
-        loss, aux = _C.softmin_loss_forward_impl(w, centers, tau, mean)
-        ctx.save_for_backward(w, centers, aux)
-        ctx.tau, ctx.mean = tau, mean
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad: Tensor):
-        w, centers, aux = ctx.saved_tensors
-        g = grad / max(1, w.numel()) if ctx.mean else grad
-        gw, gc = _C.softmin_loss_backward_impl(w, centers, ctx.tau, aux, g)
-        return gw, gc.to(centers.dtype).reshape(centers.shape), None, None
+    return _native.soft_dequantize(w, centers, _tau(tau))
 
 
 def dimq_softmin_loss(w: Tensor, centers: Tensor, tau: float, reduction: str = "sum",
@@ -110,21 +67,7 @@ def dimq_softmin_loss(w: Tensor, centers: Tensor, tau: float, reduction: str = "
         raise ValueError("centers must be non-empty")
     if reduction not in ("sum", "mean_per_layer"):
         raise ValueError(f"Unsupported loss reduction: {reduction}")
-    return _Softmin.apply(w, centers, _tau(tau), reduction == "mean_per_layer")
-
-
-class _Separation(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, w: Tensor, centers: Tensor, eta: float, eps: float) -> Tensor:
-        loss, gc = _C.separation_loss_impl(w, centers, eta, eps)
-        ctx.save_for_backward(gc)
-        ctx.shape, ctx.dtype = centers.shape, centers.dtype
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad: Tensor):
-        (gc,) = ctx.saved_tensors
-        return None, (grad * gc).to(ctx.dtype).reshape(ctx.shape), None, None
+    return _native.softmin_loss(w, centers, _tau(tau), reduction == "mean_per_layer")
 
 
 def separation_loss(w: Tensor, centers: Tensor, eta: float = 1.0, eps: float = 1e-12) -> Tensor:
@@ -132,4 +75,4 @@ def separation_loss(w: Tensor, centers: Tensor, eta: float = 1.0, eps: float = 1
     (quant/dimq.py:276-296)."""
     if centers.numel() <= 1:
         return centers.new_zeros((), dtype=torch.float32)
-    return _Separation.apply(w, centers, float(eta), float(eps))
+    return _native.separation_loss(w, centers, float(eta), float(eps))
