@@ -1,0 +1,38 @@
+"""Nearest-centre assignment: the register form (up to 8 centres) and the sorted form (16, 256) at the counts where
+one gives way to the next, aligned and unaligned rows, several trips per work-group, and centres whose gaps force the
+full scan; exact against torch's argmin."""
+
+import pytest
+import torch
+
+from tests.conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("K", [1, 4, 5, 8, 9, 16, 17, 256])
+@pytest.mark.parametrize("rows,n", [(3, 4), (2, 1025), (5, 4100), (300, 1028), (257, 7), (1, 270_001)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_nearest_centre_forms(gpu, K, rows, n, dt):
+    from dimq_amd import ops
+    announce(f"nearest K={K} rows={rows} n={n} {dt}")
+    g = torch.Generator().manual_seed(K * n)
+    cases = [torch.randn(rows, K, generator=g),
+             torch.randint(-6, 7, (rows, K), generator=g).float() * 0.25,    # duplicates and exact ties
+             torch.randn(rows, K, generator=g) * 1e-19,                      # squares below the normal range
+             1.0 + torch.randint(0, 4, (rows, K), generator=g) * 2.0 ** -23]  # gaps of an ulp, far from most weights
+    special = torch.randn(rows, K, generator=g)
+    special[0, K // 2] = float("inf")
+    special[-1, K - 1] = float("nan")
+    for c in cases + [special]:
+        w = torch.randn(rows, n, generator=g).to(dt)
+        w[0, :4] = torch.tensor([float("nan"), float("inf"), -1e30, 0.125]).to(dt)
+        idx, val = ops.hard_quantize(w.to(gpu), c.to(gpu), True)
+        for r in range(rows):
+            want = ((w[r].float()[:, None] - c[r][None, :]) ** 2).argmin(1)
+            assert torch.equal(idx[r].cpu().long(), want)
+            assert torch.equal(val[r].cpu().isnan(), c[r][want].isnan())
+            assert torch.equal(val[r].cpu().nan_to_num(), c[r][want].to(dt).nan_to_num())
+    off = torch.randn(n + 1, generator=g).to(dt).to(gpu)[1:]  # rows off the vector loads' alignment
+    idx, val = ops.hard_quantize(off, cases[0][0].to(gpu), False)
+    assert torch.equal(idx.cpu().long(), ((off.cpu().float()[:, None] - cases[0][0][None, :]) ** 2).argmin(1))
