@@ -445,6 +445,7 @@ __device__ __forceinline__ void epiN(const Epi& e, int64_t off, float (&v)[N], b
 // Combinations a kernel is not instantiated for run on the generic kernels,
 // whose epilogue is the runtime one above.
 constexpr int kEpiNone = 0, kEpiRelu = 1, kEpiGelu = 2, kEpiRes = 4, kEpiResRelu = 5, kEpiQuant = 8;
+constexpr int kEpiSplit = 16;  // no epilogue: one of several k ranges, fp32 sums for launch_split_reduce
 
 inline int epi_mode(const Epi& e) { return (e.res ? kEpiRes : 0) | e.act | (e.quant ? kEpiQuant : 0); }
 

@@ -157,6 +157,15 @@ int gemm_conv_tile(int64_t M, int64_t N, int64_t K) {
   return t128 >= device_cus() ? 0 : 1;
 }
 
+// k ranges of the implicit-GEMM conv on its 64x128 tiles, which take about
+// 0.55 us per 64-k stage: a small batch has few tiles and a long k.  C 512, 7x7,
+// 3x3 (72 stages), batch 1: 42.0 -> 16.9 us in 6 ranges, 16: 43.1 -> 22.8 in 4,
+// 32: 43.7 -> 32.0 in 3; C 256, 14x14 (36), batch 1: 23.5 -> 13.7 in 6.
+int gemm_conv_splits(int64_t M, int64_t N, int64_t K) {
+  if (gemm_conv_tile(M, N, K) != 1) return 1;
+  return split_ranges(((M + 63) / 64) * ((N + 127) / 128), K / 64, 0.55, M * N);
+}
+
 // The conv's arguments as the general pre-laid path's plan reads them (no pointers).
 GemmArgs shape_args(const ConvShape& s, int x_layout, int y_layout, int cb_dt) {
   return conv_args(s, nullptr, x_layout, nullptr, nullptr, cb_dt, 1, 1, nullptr, DIMQ_F32, nullptr, DIMQ_F32, y_layout);
@@ -483,8 +492,8 @@ static ConvPath conv_path(const ConvShape& s, int x_dtype, int x_layout, int y_d
 }
 
 // Workspace with which dimq_conv2d_codebook_ex_ws runs the general pre-laid
-// path on a call whose pointers are 16-byte aligned; 0 when another kernel
-// takes the shape.
+// path, or the implicit GEMM's k ranges, on a call whose pointers are 16-byte
+// aligned; 0 when neither takes the shape.
 extern "C" int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H,
                                                         int64_t W, int bits, int prepared, int cb_dtype,
                                                         int64_t cb_rows, int64_t cb_size, int64_t out_channels, int64_t kernel_h, int64_t kernel_w,
@@ -505,9 +514,14 @@ extern "C" int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layou
   const bool stem = stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits,
                                   x_dtype, y_dtype, al, al, mode, static_cast<const uint8_t*>(al),
                                   (s.OC * s.ICg * s.KH * s.KW * bits + 7) / 8, al, cb_dtype, cb_rows, cb_size);
-  if (conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared != 0, mode, variant, true, true, stem) !=
-      kConvGeneral)
-    return 0;
+  const ConvPath path = conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared != 0, mode, variant, true,
+                                  true, stem);
+  if (path == kConvGemm) {
+    const int64_t M = B * s.OH * s.OW;
+    const int sp = gemm_conv_splits(M, s.OC, s.ICg * s.KH * s.KW);
+    return sp > 1 ? split_bytes(sp, M, s.OC) : 0;
+  }
+  if (path != kConvGeneral) return 0;
   const GenPlan g = gen_plan(shape_args(s, x_layout, y_layout, DIMQ_F32), bits, x_dtype, false, true);
   return g.ok ? g.bytes : 0;
 }
@@ -562,6 +576,20 @@ extern "C" int dimq_conv2d_codebook_ex_ws(const void* x, int x_dtype, int x_layo
     p.ldy = s.OC;
     p.epi = epi;
     const int tile = gemm_conv_tile(p.M, p.N, p.K);
+    if (const int sp = gemm_conv_splits(p.M, p.N, p.K);
+        sp > 1 && workspace != nullptr && aligned(workspace, 256) && workspace_bytes >= split_bytes(sp, p.M, p.ldy)) {
+      const GemmArgs q = split_args(p, sp, workspace);
+      int rs = DIMQ_OK;
+      switch (bits) {
+        case 2: rs = launch_big_conv_b2(q, x_dtype, 1, as_stream(stream)); break;
+        case 3: rs = launch_big_conv_b3(q, x_dtype, 1, as_stream(stream)); break;
+        default: rs = launch_big_conv_b4(q, x_dtype, 1, as_stream(stream)); break;
+      }
+      if (rs != DIMQ_OK) return rs;
+      launch_split_reduce(p, static_cast<const float*>(workspace), sp, nullptr, x_dtype, bits, x_dtype != DIMQ_F16,
+                          true, as_stream(stream));
+      return check_launch("conv2d_codebook (split k)");
+    }
     switch (bits) {
       case 2: return launch_big_conv_b2(p, x_dtype, tile, as_stream(stream));
       case 3: return launch_big_conv_b3(p, x_dtype, tile, as_stream(stream));

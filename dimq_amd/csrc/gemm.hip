@@ -32,9 +32,12 @@ int gemm_fast_tile(int tile, const GemmArgs& p, int bits) {
 }
 
 // Large-tile kernels (gemm_big.h) for Linear shapes with M > 64, K % 64 == 0
-// and aligned rows/streams.  Measured on the ViT-B/16 shapes (M = 12,608) and
-// cfg1: the deep-pipeline tile (7, 64x128) is fastest for K < 2048, the 2x2
-// 128x128 tile (2) for K >= 2048.  Returns -1 when the shape does not qualify.
+// and aligned rows/streams.  The deep-pipeline tile (7, 64x128) is fastest
+// below 2,048 rows (128x128 tile against it at M 100, N = K = 4,096: 62 and 45
+// us; M 500: 61 and 41; M 1,024: 69 and 61; M 1,576, N 768, K 3,072: 47 and 31;
+// M 2,047, N 3,072, K 2,304: 53 and 49); the 2x2 128x128 tile (2) for long k
+// and fp32 activations above (M 12,608, K 3,072).  Returns -1 when the shape
+// does not qualify.
 int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
   if (variant == DIMQ_VARIANT_SMALL_M || p.conv || !(bits == 2 || bits == 3 || bits == 4)) return -1;
   const int mode = epi_mode(p.epi);  // epilogues the large tiles are instantiated for
@@ -47,7 +50,7 @@ int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
   // 133 against the best 128x128 tile); below M 2048 the 128x128 tiles fill
   // the CUs better (M 1000: 17 vs 30 us).
   if (p.M >= 2048 && x_dtype != DIMQ_F32) return 10;  // fp32 activations spill its registers
-  return p.K >= 2048 ? 2 : 7;
+  return p.M >= 2048 && p.K >= 2048 ? 2 : 7;
 }
 
 // Whether the general pre-laid path (gemm_gen.hip) takes a Linear that no path
@@ -62,6 +65,16 @@ bool gen_wants_linear(int64_t M, int64_t K, int64_t N, int bits) {
   if (M <= 16) return false;
   if (bits == 8 || K % 64 != 0) return true;
   return M <= 64 && (K % 128 != 0 || (K >= 1024 && N * K <= (8ll << 20)));
+}
+
+// k ranges of a Linear on the 64x128 tiles.  A 64-k stage takes 0.45 us there.
+// M 197, N 768, K 3,072 (24 tiles): 29.3 -> 16.2 us in 6 ranges; M 788: 29.6 ->
+// 21.3 in 3; M 100, N = K = 4,096: 45.1 -> 22.5 in 4.  At K < 2,048 the second
+// launch costs what the ranges save (M 197, N = K = 768: 12.9 against 12.2 to
+// 14.0), and at M 500, N = K = 4,096 the tiles fill the chip (41.4, 41.0).
+int big_linear_splits(int64_t M, int64_t K, int64_t N, int tile) {
+  if (tile != 7 || K < 2048) return 1;
+  return split_ranges(((M + 63) / 64) * ((N + 127) / 128), K / 64, 0.45, M * N);
 }
 
 int gemm_pick_tile(int64_t M, int64_t N, int variant) {
@@ -147,6 +160,22 @@ int linear_codebook_impl(const void* x, int x_dtype, int64_t M, int64_t K, int64
       aligned(workspace, 256) && variant != DIMQ_VARIANT_SMALL_M) {
     const GenPlan g = gen_plan(p, bits, x_dtype, false, aligned(x, 16));
     if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, bits, x_dtype, workspace, s);
+  }
+  if (big >= 0 && workspace != nullptr && aligned(workspace, 256)) {
+    const int sp = big_linear_splits(M, K, N, big);
+    if (sp > 1 && workspace_bytes >= split_bytes(sp, M, ldy)) {
+      const GemmArgs q = split_args(p, sp, workspace);
+      int rc = DIMQ_OK;
+      switch (bits) {
+        case 2: rc = launch_big_b2(q, x_dtype, big, s); break;
+        case 3: rc = launch_big_b3(q, x_dtype, big, s); break;
+        default: rc = launch_big_b4(q, x_dtype, big, s); break;
+      }
+      if (rc != DIMQ_OK) return rc;
+      launch_split_reduce(p, static_cast<const float*>(workspace), sp, nullptr, x_dtype, bits, x_dtype != DIMQ_F16,
+                          false, s);
+      return check_launch("linear_codebook (split k)");
+    }
   }
   if (big >= 0) {
     switch (bits) {
@@ -234,11 +263,16 @@ static GemmArgs linear_shape_args(int64_t M, int64_t K, int64_t N, int cb_dtype)
   return p;
 }
 
-// dimq_linear_codebook_workspace_bytes, or what the general pre-laid path
-// needs where no other path with a workspace takes the shape.
+// dimq_linear_codebook_workspace_bytes, or what the general pre-laid path or
+// the partial outputs of the large tiles' k ranges need where no other path
+// with a workspace takes the shape.
 extern "C" int64_t dimq_linear_codebook_full_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype) {
   const int64_t own = dimq_linear_codebook_workspace_bytes(M, K, N, bits, x_dtype);
-  if (own > 0 || M <= 0 || K <= 0 || N <= 0 || !gen_wants_linear(M, K, N, bits)) return own;
+  if (own > 0 || M <= 0 || K <= 0 || N <= 0) return own;
+  if (!gen_wants_linear(M, K, N, bits)) {
+    const int sp = M > 64 && M < 2048 ? big_linear_splits(M, K, N, 7) : 1;
+    return sp > 1 ? split_bytes(sp, M, N) : 0;
+  }
   const GenPlan g = gen_plan(linear_shape_args(M, K, N, DIMQ_F32), bits, x_dtype, false, true);
   return g.ok ? g.bytes : 0;
 }

@@ -165,6 +165,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
   tile_coords((p.N + BN - 1) / BN, mt, nt);
   const int64_t m0 = mt * BM;
   const int64_t n0 = nt * BN;
+  constexpr bool SPLIT = (MODE & kEpiSplit) != 0;
+  void* const yb = SPLIT ? static_cast<void*>(static_cast<float*>(p.y) + blockIdx.y * (p.M * p.ldy)) : p.y;
 
   stage_codebook<E>(p.cb, p.cb_dt, p.cb_rows, p.cb_size, n0, BN, p.N, cbs, tid, NT);
   for (int c = tid; c < BN; c += NT) ebias[c] = (p.bias && n0 + c < p.N) ? load_as_float(p.bias, p.bias_dt, n0 + c) : 0.0f;
@@ -222,7 +224,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.0f;
 
-  const int64_t nk = p.K / kBigKS;
+  const int64_t nka = p.K / kBigKS;
+  const int64_t kfirst = SPLIT ? nka * blockIdx.y / p.splits : 0;  // the work-group's stages: nk from kfirst
+  const int64_t nk = SPLIT ? nka * (blockIdx.y + 1) / p.splits - kfirst : nka;
   RawA<XT> ra[A_TASKS];
   bool avalid[A_TASKS];  // CONV: the task's tap lies inside the image (else its group reads as zeros)
   uint32_t b0[NBLK][2 * BITS], b1[NBLK][2 * BITS];
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
   // being computed then also waited for part of the next stage's loads,
   // issued just before (a full memory latency per 64-k stage).
   auto issue_a = [&](int64_t kt) {
-    const int64_t k = (kt < nk ? kt : nk - 1) * kBigKS;
+    const int64_t k = (kfirst + (kt < nk ? kt : nk - 1)) * kBigKS;
     if constexpr (CONV) {
       const int tap = static_cast<int>(k / p.cC);
       const int64_t c0 = k - tap * p.cC;
@@ -264,14 +268,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
 #pragma unroll
         for (int w = 0; w < 8; ++w) o[w] &= m;
       }
-      if (range_guarded<XT>() && track) trk = range_track(trk, o);
+      if (range_guarded<XT>() && (SPLIT || track)) trk = range_track(trk, o);
       uint4* dst = reinterpret_cast<uint4*>(&As[buf][alds[i]]);
       dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
       dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
     }
   };
   auto issue_b = [&](int64_t kt, uint32_t (&dst)[NBLK][2 * BITS]) {
-    const int64_t k = (kt < nk ? kt : nk - 1) * kBigKS;
+    const int64_t k = (kfirst + (kt < nk ? kt : nk - 1)) * kBigKS;
 #pragma unroll
     for (int nb = 0; nb < NBLK; ++nb) issue_b_stage<BITS>(p.w, brow[nb], p.K, k, dst[nb]);
   };
@@ -331,7 +335,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
   // commit, which waits for them, after the MFMAs.
   issue_a(0);
   issue_b(0, b0);
-  commit_a(0, true);  // the range guard looks at the first k stage
+  commit_a(0, true);  // the range guard looks at the first k stage (SPLIT: at all, any may start a range)
   __syncthreads();
   int64_t kt = 0;
   for (; kt + 2 <= nk; kt += 2) {
@@ -354,8 +358,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
 
   if constexpr (range_guarded<XT>()) {
     if (tile_needs_exact(p, XT, m0, m0 + BM, trk, finite_acc<1>(&acc[0][0], MBLK, NBLK))) {
-      exact_tile_out(p, XT, BITS, m0, m0 + BM, n0, n0 + BN, 0, CONV);
-      return;
+      if constexpr (SPLIT) {  // NaN partial sums: the second pass recomputes what they reach
+#pragma unroll
+        for (int mb = 0; mb < MBLK; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < NBLK; ++nb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = __builtin_nanf("");
+      } else {
+        exact_tile_out(p, XT, BITS, m0, m0 + BM, n0, n0 + BN, 0, CONV);
+        return;
+      }
     }
   }
 
@@ -384,7 +397,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
     constexpr int CPT = (CH + NT - 1) / NT;  // chunks per thread
     static_assert(NT % (PW / 8) == 0, "a thread's chunks share one column group");
     float* ot = reinterpret_cast<float*>(&As[0][0]);
-    const bool vec8 = p.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.y_dt != DIMQ_F64;
+    const bool vec8 = p.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(yb) & 15) == 0 && p.y_dt != DIMQ_F64;
     const int qg = tid % (PW / 8);  // this thread's 8-column group of every pass
     const bool rpair = (MODE & kEpiRes) && res_pairs(p.epi, vec8);
     auto res_load = [&](int nb, ResPairs<8> (&rr)[CPT]) {
@@ -441,7 +454,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
         if (vec8 && n + 8 <= p.N) {
           epi_m<MODE, 8>(p.epi, &rr[u], off, true, v[u]);
           if (p.y_dt == DIMQ_F32) {
-            f4v* yp = reinterpret_cast<f4v*>(reinterpret_cast<float*>(p.y) + off);
+            f4v* yp = reinterpret_cast<f4v*>(reinterpret_cast<float*>(yb) + off);
             const f4v lo = {v[u][0], v[u][1], v[u][2], v[u][3]}, hi = {v[u][4], v[u][5], v[u][6], v[u][7]};
             yp[0] = lo;
             yp[1] = hi;
@@ -454,12 +467,12 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
 #pragma unroll
               for (int i = 0; i < 4; ++i) h[i] = bf16x2_rne(v[u][2 * i], v[u][2 * i + 1]);
             }
-            u32x4* yp = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.y) + off);
+            u32x4* yp = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(yb) + off);
             *yp = h;
           }
         } else {
           for (int i = 0; i < 8; ++i)
-            if (n + i < p.N) store_from_float(p.y, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[u][i]));
+            if (n + i < p.N) store_from_float(yb, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[u][i]));
         }
       }
       __syncthreads();  // the next pass overwrites the parked values
@@ -475,7 +488,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
     // values, so lane g holds the 8 columns 16 jp + 8 g .. + 7 of its row and
     // writes them as one 16-byte store (two 8-byte stores per lane before).
     const bool vec = p.ldy % 4 == 0 && p.y_dt != DIMQ_F64;
-    const bool vec8 = p.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.y_dt != DIMQ_F64;
+    const bool vec8 = p.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(yb) & 15) == 0 && p.y_dt != DIMQ_F64;
     // 16-bit residuals of row group gi = 2 nb + jp, requested one group ahead
     // of its stores (two register sets; a whole-tile prefetch would cost this
     // kernel an occupancy step), so each group's loads land during the
@@ -538,7 +551,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
             if (n8 + 8 <= p.N) {
               epi_m<MODE, 8>(p.epi, &rr[mb], off, true, v);
               if (p.y_dt == DIMQ_F32) {
-                float* yp = reinterpret_cast<float*>(p.y) + off;
+                float* yp = reinterpret_cast<float*>(yb) + off;
                 *reinterpret_cast<float4*>(yp) = make_float4(v[0], v[1], v[2], v[3]);
                 *reinterpret_cast<float4*>(yp + 4) = make_float4(v[4], v[5], v[6], v[7]);
               } else {
@@ -546,11 +559,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                   h[i] = p.y_dt == DIMQ_F16 ? f16x2_rne(v[2 * i], v[2 * i + 1]) : bf16x2_rne(v[2 * i], v[2 * i + 1]);
-                *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.y) + off) = make_uint4(h[0], h[1], h[2], h[3]);
+                *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(yb) + off) = make_uint4(h[0], h[1], h[2], h[3]);
               }
             } else {
               for (int i = 0; i < 8; ++i)
-                if (n8 + i < p.N) store_from_float(p.y, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[i]));
+                if (n8 + i < p.N) store_from_float(yb, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[i]));
             }
           } else {
             if (m >= p.M) continue;
@@ -563,15 +576,15 @@ __global__ __launch_bounds__(64 * WGM * WGN, big_min_waves(BITS, MBLK, NBLK, CON
               if (vec && n + 4 <= p.N) {
                 epi_m<MODE, 4>(p.epi, nullptr, off, true, v);
                 if (p.y_dt == DIMQ_F32) {
-                  *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.y) + off) = make_float4(v[0], v[1], v[2], v[3]);
+                  *reinterpret_cast<float4*>(reinterpret_cast<float*>(yb) + off) = make_float4(v[0], v[1], v[2], v[3]);
                 } else {
                   const uint32_t h0 = p.y_dt == DIMQ_F16 ? f16x2_rne(v[0], v[1]) : bf16x2_rne(v[0], v[1]);
                   const uint32_t h1 = p.y_dt == DIMQ_F16 ? f16x2_rne(v[2], v[3]) : bf16x2_rne(v[2], v[3]);
-                  *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.y) + off) = make_uint2(h0, h1);
+                  *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(yb) + off) = make_uint2(h0, h1);
                 }
               } else {
                 for (int i = 0; i < 4; ++i)
-                  if (n + i < p.N) store_from_float(p.y, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[i]));
+                  if (n + i < p.N) store_from_float(yb, p.y_dt, off + i, epi1_m<MODE>(p.epi, off + i, v[i]));
               }
             }
           }
@@ -1178,6 +1191,19 @@ int launch_big(const GemmArgs& p, hipStream_t s) {
   return check_launch(CONV ? "conv2d_codebook (implicit GEMM, large tiles)" : "linear_codebook (large tiles)");
 }
 
+// p.splits k ranges (few tiles, long k) on 64x128 tiles, one wave per 32
+// columns: as fast or faster than 128x128 in 2 to 8 ranges at 14 Linear shapes
+// (M 100, N = K = 4,096, 4 ranges: 17.1 against 23.6 us).
+template <int BITS, int XT, int WGM, int WGN, int MBLK, int NBLK, bool CONV>
+int launch_big_split(const GemmArgs& p, hipStream_t s) {
+  constexpr int BM = WGM * MBLK * 32, BN = WGN * NBLK * 32;
+  const int64_t tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  hipLaunchKernelGGL((gemm_big_kernel<BITS, XT, WGM, WGN, MBLK, NBLK, CONV, kEpiSplit>),
+                     dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(p.splits)), dim3(64 * WGM * WGN), 0, s,
+                     p);
+  return check_launch("codebook GEMM (large tiles, split k)");
+}
+
 // Implicit-GEMM conv tiles: 0 = 128x128 (2x2 waves of 64x64), 1 = 64x128
 // (1x4 waves of 64x32), 2 = 256x128 (2x2 waves of 128x64).
 // Epilogue modes: none / relu / residual / residual + relu on tiles 0 and 1
@@ -1197,6 +1223,9 @@ int launch_big_conv_modes(const GemmArgs& p, int mode, hipStream_t s) {
 template <int BITS>
 int launch_big_conv_bits(const GemmArgs& p, int xt, int tile, hipStream_t s) {
   const int mode = epi_mode(p.epi);
+  if (p.splits > 1)
+    return xt == DIMQ_F16 ? launch_big_split<BITS, DIMQ_F16, 1, 4, 2, 1, true>(p, s)
+                          : launch_big_split<BITS, DIMQ_BF16, 1, 4, 2, 1, true>(p, s);
 #define DIMQ_CONV_TILES(XT)                                                 \
   switch (tile) {                                                           \
     case 1: return launch_big_conv_modes<BITS, XT, 1, 4, 2, 1>(p, mode, s); \
@@ -1217,6 +1246,7 @@ int launch_big_conv_bits(const GemmArgs& p, int xt, int tile, hipStream_t s) {
 // activation quantization.
 template <int BITS, int XT>
 int launch_big_linear_modes(const GemmArgs& p, int tile, int mode, hipStream_t s) {
+  if (p.splits > 1) return launch_big_split<BITS, XT, 1, 4, 2, 1, false>(p, s);
   if constexpr (XT == DIMQ_F16) {
     if ((mode & kEpiQuant) != 0) {
       switch (mode) {

@@ -39,4 +39,19 @@ int split_ranges(int64_t tiles, int64_t stages, double us_per_stage, int64_t out
 void launch_split_reduce(const GemmArgs& p, const float* part, int splits, const float* rs, int x_dtype, int bits,
                          bool guard, bool tapmajor, hipStream_t s);
 
+// The two launches of a split codebook GEMM on gemm_big_kernel: the arguments
+// of the first, and the workspace of its partial outputs.
+inline int64_t split_bytes(int splits, int64_t M, int64_t ldy) {
+  return (static_cast<int64_t>(splits) * M * ldy * 4 + 255) / 256 * 256;
+}
+inline GemmArgs split_args(const GemmArgs& p, int splits, void* ws) {
+  GemmArgs q = p;
+  q.splits = splits;
+  q.y = ws;
+  q.y_dt = DIMQ_F32;
+  q.bias = nullptr;
+  q.epi = Epi{};
+  return q;
+}
+
 }  // namespace dimq

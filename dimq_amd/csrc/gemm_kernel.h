@@ -55,6 +55,9 @@ struct GemmArgs {
   // the activation scale of a W4A4 call whose activations were pre-quantized
   // to the exact fp16 integers a - zp
   float acc_scale = 1.0f;
+  // gemm_big_kernel with kEpiSplit: k range blockIdx.y of `splits`; y is that
+  // many fp32 planes of M * ldy, bias and epilogue are the second pass's
+  int splits = 1;
 };
 
 // Output element offset of (row m, global column n).

@@ -316,7 +316,8 @@ int dimq_linear_codebook_ex(const void* x, int x_dtype, int64_t M, int64_t K, co
  * be ordered on it. */
 int64_t dimq_linear_codebook_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype);
 /* The same, or for shapes without such a path (8-bit codebooks, in_features
- * off the k steps, 16 < M <= 64) the general pre-laid path's workspace. */
+ * off the k steps, 16 < M <= 64) the general pre-laid path's workspace, or
+ * (64 < M < 2048, few tiles, long k) the fp32 partial outputs of the k ranges. */
 int64_t dimq_linear_codebook_full_workspace_bytes(int64_t M, int64_t K, int64_t N, int bits, int x_dtype);
 int dimq_linear_codebook_ex_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint8_t* packed_w,
                                int64_t packed_numel, int bits, const void* codebook, int cb_dtype, int64_t cb_rows,
@@ -435,7 +436,8 @@ int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout, int64_t B,
  * kernels' forms, groups, dilation, 8-bit, odd channel counts) lay weights and
  * activations out in it as fp16 and run the general pre-laid path, when it
  * holds dimq_conv2d_codebook_workspace_bytes (0: another kernel takes the
- * call).  `prepared`, `residual`: whether the call passes one. */
+ * call); the implicit GEMM on a prepared weight keeps the fp32 partial outputs
+ * of its k ranges there when it has few tiles.  `prepared`, `residual`: whether the call passes one. */
 int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H, int64_t W,
                                              int bits, int prepared, int cb_dtype, int64_t cb_rows, int64_t cb_size,
                                              int64_t out_channels, int64_t kernel_h, int64_t kernel_w,
