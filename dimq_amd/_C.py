@@ -533,10 +533,11 @@ build_product_table = build_product_table_impl
 
 
 def linear_lut(x, packed_w, codebook, act_scale, act_zp, bias, out_features, in_features):
-    return _native.linear_lut(x, packed_w, codebook, act_scale, act_zp, bias, out_features, in_features)
+    return _native.linear_lut(x, packed_w, codebook, float(act_scale), int(act_zp), bias, out_features, in_features)
 
 
 def conv2d_lut(x, packed_w, codebook, act_scale, act_zp, bias, out_channels, in_channels_per_group, kernel_h, kernel_w,
                stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, groups):
-    return _native.conv2d_lut(x, packed_w, codebook, act_scale, act_zp, bias, out_channels, in_channels_per_group,
-                              kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, groups)
+    return _native.conv2d_lut(x, packed_w, codebook, float(act_scale), int(act_zp), bias, out_channels,
+                              in_channels_per_group, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w, dilation_h,
+                              dilation_w, groups)
