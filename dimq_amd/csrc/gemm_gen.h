@@ -14,7 +14,8 @@ struct GenPlan {
   int splits = 1;         // k ranges (> 1: fp32 partial outputs and a second pass)
   int64_t cg = 0;         // channels per group padded to 8 (Linear: K padded to a stage)
   int64_t kp = 0;         // k of one weight plane: taps * cg, padded to a stage
-  int64_t pixels = 0;     // rows of the laid-out activations
+  int64_t step = 0;       // images (Linear: rows) laid out and multiplied at a time
+  int64_t pixels = 0;     // rows of the laid-out activations: those of `step` images
   int64_t planes = 0;     // flag words per row (0: fp16 activations or codes, no range guard)
   int64_t off_rs = 0, off_x = 0, off_flags = 0, off_zero = 0, off_part = 0;
   int64_t bytes = 0;      // workspace

@@ -37,6 +37,13 @@ constexpr int kGenS = 3;              // slots of the LDS ring
 constexpr int kGenRows = 4;           // weight rows per work-group of the first launch, one per wave
 constexpr int kGenRaw = 16384;        // packed bytes of a work-group's rows kept in LDS
 constexpr int kGenPix = 64, kGenChan = 64;  // pixels x channels of an NCHW transpose work-group
+// Laid-out activations and flags of a call in its workspace: larger ones go in
+// several passes of whole images (Linear: rows) over the same workspace.  A
+// depthwise layer's channels are padded eightfold, so its layout is 8 to 10
+// times an fp16 input: 128 x 96 x 112 x 112, 3x3, needed 2.87 GiB in one pass.
+// That layer takes 28.1 ms in ten passes (fp16, channels last; 29.3 in one, 257
+// on gemm_cb_kernel) and 22.2 in 12 (fp32 NCHW; 22.3, 273).
+constexpr int64_t kGenActBytes = 256ll << 20;
 
 // Chunk c of stage row r lies at 128 r + ((c ^ gen_swz(r)) << 4), so that the
 // 16 rows of one 16-byte LDS read cover all 64 banks.
@@ -742,8 +749,18 @@ GenPlan gen_plan(const GemmArgs& p, int bits, int x_dtype, bool a4, bool in_plac
   const int64_t cpl = cdiv(g.cg, kGenChan);
   const bool guard = !a4 && (x_dtype == DIMQ_F32 || x_dtype == DIMQ_BF16);
   g.planes = guard ? groups * cpl : 0;
+  const int64_t units = g.conv ? p.cB : p.M;  // images, or rows
+  const int64_t unit_bytes = g.pixels / units * ((g.direct_x ? 0 : xpitch * 2) + g.planes * 4);
+  g.step = units;
+  if (units * unit_bytes > kGenActBytes) {
+    const int64_t most = unit_bytes < kGenActBytes ? kGenActBytes / unit_bytes : 1;
+    g.step = cdiv(units, cdiv(units, most));  // passes of about the same size
+    if (!g.conv && most >= kGenB) g.step = cdiv(g.step, kGenB) * kGenB <= most ? cdiv(g.step, kGenB) * kGenB : most / kGenB * kGenB;
+    g.pixels = g.pixels / units * g.step;
+  }
+  const int64_t M = p.M / units * g.step;  // rows of a pass
   // a 64-k stage takes about 0.3 us on a CU of its own
-  g.splits = split_ranges(cdiv(p.M, kGenB) * cdiv(p.N, kGenB) * groups, nk, 0.3, p.M * p.N * groups);
+  g.splits = split_ranges(cdiv(M, kGenB) * cdiv(p.N, kGenB) * groups, nk, 0.3, M * p.N * groups);
   int64_t at = up256(rows * ldw * 2);
   g.off_rs = at;
   at += up256(rows * 4);
@@ -759,7 +776,7 @@ GenPlan gen_plan(const GemmArgs& p, int bits, int x_dtype, bool a4, bool in_plac
   }
   if (g.splits > 1) {
     g.off_part = at;
-    at += up256(static_cast<int64_t>(g.splits) * p.M * (g.conv ? p.cOC : p.ldy) * 4);
+    at += up256(static_cast<int64_t>(g.splits) * M * (g.conv ? p.cOC : p.ldy) * 4);
   }
   g.bytes = at;
   g.ok = true;
@@ -788,31 +805,47 @@ int launch_gen(const GemmArgs& p, const GenPlan& g, int bits, int x_dtype, void*
   a.cg = g.cg;
   a.kp = g.kp;
   a.ldw = g.kp * (g.hilo ? 2 : 1);
-  a.pixels = g.pixels;
   a.planes = g.planes;
   a.cpl = cdiv(g.cg, kGenChan);
-  a.xa = g.direct_x ? static_cast<const uint16_t*>(p.x) : a.xh;
   a.xpitch = static_cast<uint32_t>(g.direct_x ? (g.conv ? p.cC : p.ldx) : groups * g.cg);
   a.xgroup = static_cast<uint32_t>(g.direct_x ? a.icg : g.cg);
   a.splits = g.splits;
-  int64_t nbx = 0;
-  if (a.xmode == 0) nbx = cdiv(g.pixels, kGenPix) * groups * a.cpl;
-  if (a.xmode == 1) nbx = cdiv(g.pixels * groups * a.cpl, 32);
-  const dim3 grid(static_cast<unsigned>(a.nbw + nbx));
-  switch (bits) {
-    case 2: hipLaunchKernelGGL(gen_prep_kernel<2>, grid, dim3(256), 0, s, p, a); break;
-    case 3: hipLaunchKernelGGL(gen_prep_kernel<3>, grid, dim3(256), 0, s, p, a); break;
-    case 4: hipLaunchKernelGGL(gen_prep_kernel<4>, grid, dim3(256), 0, s, p, a); break;
-    default: hipLaunchKernelGGL(gen_prep_kernel<8>, grid, dim3(256), 0, s, p, a); break;
-  }
-  const int rc = check_launch("codebook layer (operand layout)");
-  if (rc != DIMQ_OK) return rc;
-  if (g.conv) {
-    if (g.planes) launch_gen_gemm<true, true>(p, a, bits, s);
-    else launch_gen_gemm<true, false>(p, a, bits, s);
-  } else {
-    if (g.planes) launch_gen_gemm<false, true>(p, a, bits, s);
-    else launch_gen_gemm<false, false>(p, a, bits, s);
+  const int64_t units = g.conv ? p.cB : p.M;
+  const int64_t unit_m = p.M / units, unit_pixels = g.pixels / g.step;
+  const int64_t unit_x = g.conv ? p.cC * p.cH * p.cW : p.ldx, unit_y = unit_m * (g.conv ? p.cOC : p.ldy);
+  for (int64_t u = 0; u < units; u += g.step) {
+    const int64_t n = units - u < g.step ? units - u : g.step;
+    GemmArgs q = p;  // this pass's images: x, y and the residual all have them outermost
+    q.x = static_cast<const uint8_t*>(p.x) + u * unit_x * dtype_size(x_dtype);
+    q.y = static_cast<uint8_t*>(p.y) + u * unit_y * dtype_size(p.y_dt);
+    if (p.epi.res) {
+      q.epi.res = static_cast<const uint8_t*>(p.epi.res) + u * unit_y * dtype_size(p.epi.res_dt);
+      q.epi.res_vec = aligned(q.epi.res, 16);
+    }
+    q.M = n * unit_m;
+    if (g.conv) q.cB = n;
+    a.pixels = n * unit_pixels;
+    a.xa = g.direct_x ? static_cast<const uint16_t*>(q.x) : a.xh;
+    if (u > 0) a.nbw = 0;  // the weights are laid out
+    int64_t nbx = 0;
+    if (a.xmode == 0) nbx = cdiv(a.pixels, kGenPix) * groups * a.cpl;
+    if (a.xmode == 1) nbx = cdiv(a.pixels * groups * a.cpl, 32);
+    const dim3 grid(static_cast<unsigned>(a.nbw + nbx));
+    switch (bits) {
+      case 2: hipLaunchKernelGGL(gen_prep_kernel<2>, grid, dim3(256), 0, s, q, a); break;
+      case 3: hipLaunchKernelGGL(gen_prep_kernel<3>, grid, dim3(256), 0, s, q, a); break;
+      case 4: hipLaunchKernelGGL(gen_prep_kernel<4>, grid, dim3(256), 0, s, q, a); break;
+      default: hipLaunchKernelGGL(gen_prep_kernel<8>, grid, dim3(256), 0, s, q, a); break;
+    }
+    const int rc = check_launch("codebook layer (operand layout)");
+    if (rc != DIMQ_OK) return rc;
+    if (g.conv) {
+      if (g.planes) launch_gen_gemm<true, true>(q, a, bits, s);
+      else launch_gen_gemm<true, false>(q, a, bits, s);
+    } else {
+      if (g.planes) launch_gen_gemm<false, true>(q, a, bits, s);
+      else launch_gen_gemm<false, false>(q, a, bits, s);
+    }
   }
   return check_launch("codebook layer");
 }

@@ -436,8 +436,9 @@ int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout, int64_t B,
  * kernels' forms, groups, dilation, 8-bit, odd channel counts) lay weights and
  * activations out in it as fp16 and run the general pre-laid path, when it
  * holds dimq_conv2d_codebook_workspace_bytes (0: another kernel takes the
- * call); the implicit GEMM on a prepared weight keeps the fp32 partial outputs
- * of its k ranges there when it has few tiles.  `prepared`, `residual`: whether the call passes one. */
+ * call; the activations take at most 256 MiB of it, or one image, larger inputs
+ * going through in passes); the implicit GEMM on a prepared weight keeps the
+ * fp32 partial outputs of its k ranges there when it has few tiles.  `prepared`, `residual`: whether the call passes one. */
 int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layout, int64_t B, int64_t C, int64_t H, int64_t W,
                                              int bits, int prepared, int cb_dtype, int64_t cb_rows, int64_t cb_size,
                                              int64_t out_channels, int64_t kernel_h, int64_t kernel_w,

@@ -15,3 +15,25 @@ def test_lut_callables_take_any_real_scale_and_zero_point(scale, zp):
         _C.linear_lut(torch.zeros(1, 4), pw, cb, scale, zp, None, 1, 4)
     with pytest.raises(RuntimeError, match="conv2d_lut expects CUDA input"):
         _C.conv2d_lut(torch.zeros(1, 4, 1, 1), pw, cb, scale, zp, None, 1, 4, 1, 1, 1, 1, 0, 0, 1, 1, 1)
+
+
+def _conv_ws(x_dtype, layout, B, C, H, W, OC, ks, groups, bits=4):
+    from dimq_amd import _C
+    return _C.lib.dimq_conv2d_codebook_workspace_bytes(x_dtype, layout, B, C, H, W, bits, 0, 0, OC, 1 << bits, OC, ks, ks,
+                                                       1, 1, ks // 2, ks // 2, 1, 1, groups, x_dtype, layout, 0, 0, 0)
+
+
+def test_general_path_workspace_is_bounded():
+    """Laid-out activations and flags take at most 256 MiB however large the input: a depthwise layer's would be 8 to 10
+    times its fp16 input (2.87 GiB for the first)."""
+    from dimq_amd import _C
+    limit, weights = 256 << 20, 1 << 20
+    for dt in (_C.F32, _C.F16, _C.BF16):
+        for layout in (_C.NCHW, _C.NHWC):
+            assert 0 < _conv_ws(dt, layout, 128, 96, 112, 112, 96, 3, 96) <= limit + weights
+    lut = _C.lib.dimq_conv2d_lut_full_workspace_bytes
+    assert 0 < lut(_C.F32, 128, 96, 112, 112, 96, 1, 3, 3, 1, 1, 1, 1, 1, 1, 96, _C.F32) <= limit + weights
+    lin = _C.lib.dimq_linear_codebook_full_workspace_bytes
+    assert 0 < lin(20_000_000, 3, 16, 4, _C.F32) <= limit + weights
+    # one image beyond the bound goes by itself
+    assert limit < _conv_ws(_C.F32, _C.NCHW, 2, 64, 640, 640, 64, 3, 64) <= 640 * 640 * 64 * 20 + weights
