@@ -62,6 +62,16 @@ Tensor workspace(int64_t bytes, const Tensor& like) {
   return bytes > 0 ? at::empty({bytes}, like.options().dtype(at::kByte)) : Tensor();
 }
 
+// The workspace of a layer whose entry point has kernels that need none:
+// without room for it the call runs on those (slower) instead of failing.
+Tensor spare_workspace(int64_t bytes, const Tensor& like) {
+  try {
+    return workspace(bytes, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
+
 struct Bias {
   Tensor t;
   void* p = nullptr;
@@ -139,7 +149,7 @@ Tensor linear_lut(const Tensor& x, const Tensor& packed_w, const Tensor& codeboo
   const Bias b(bias, out_features, "out_features");
   const int64_t M = xc.numel() / in_features;
   const Tensor y = at::empty(out_shape(x, out_features), x.options().dtype(at::kFloat));
-  const Tensor ws = workspace(
+  const Tensor ws = spare_workspace(
       dimq_linear_lut_full_workspace_bytes(dt(xc), M, out_features, in_features, dt(cb)), xc);
   const On on(xc);
   check_rc(dimq_linear_lut_ws(ptr(xc), dt(xc), M, u8(pw), pw.numel(), ptr(cb), dt(cb), cb.numel(), act_scale, act_zp,
@@ -166,7 +176,7 @@ Tensor conv2d_lut(const Tensor& x, const Tensor& packed_w, const Tensor& codeboo
                               conv_out(W, pad_w, dilation_w, kernel_w, stride_w)}, x.options().dtype(at::kFloat));
   Tensor ws;
   if (y.numel() > 0)
-    ws = workspace(dimq_conv2d_lut_full_workspace_bytes(
+    ws = spare_workspace(dimq_conv2d_lut_full_workspace_bytes(
         dt(xc), B, C, H, W, out_channels, in_channels_per_group, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
         dilation_h, dilation_w, groups, dt(cb)), xc);
   const On on(xc);
@@ -196,7 +206,8 @@ Tensor linear_codebook(const Tensor& x, const Tensor& packed_w, const Tensor& co
   const Tensor y = at::empty(shape, x.options().dtype(out_dtype.value_or(x.scalar_type())));
   const Residual r(residual, shape, at::MemoryFormat::Contiguous);
   const int nb = static_cast<int>(bits), act = static_cast<int>(activation), var = static_cast<int>(variant);
-  const Tensor ws = workspace(dimq_linear_codebook_full_workspace_bytes(M, in_features, out_features, nb, dt(xc)), xc);
+  const Tensor ws =
+      spare_workspace(dimq_linear_codebook_full_workspace_bytes(M, in_features, out_features, nb, dt(xc)), xc);
   const int64_t wsn = ws.defined() ? ws.numel() : 0;
   const On on(xc);
   if (!decoded) {
@@ -244,7 +255,7 @@ Tensor conv2d_codebook(const Tensor& x, const Tensor& packed_w, const Tensor& co
   const int64_t prep_words = prep.defined() ? prep.numel() : 0;
   const Residual r(residual, y.sizes(), mf);
   const int nb = static_cast<int>(bits), act = static_cast<int>(activation), var = static_cast<int>(variant);
-  const Tensor ws = workspace(dimq_conv2d_codebook_workspace_bytes(
+  const Tensor ws = spare_workspace(dimq_conv2d_codebook_workspace_bytes(
       dt(xc), layout, B, C, H, W, nb, prep_words > 0, dt(cb), rows, size, out_channels, kernel_h, kernel_w, stride_h,
       stride_w, pad_h, pad_w, dilation_h, dilation_w, groups, dt(y), layout, r.p != nullptr, act, var), xc);
   const On on(xc);
