@@ -23,16 +23,7 @@ using OptTensor = std::optional<Tensor>;
 
 void check_rc(int rc) { TORCH_CHECK(rc == DIMQ_OK, dimq_last_error()); }
 
-std::string dtype_name(at::ScalarType t) {
-  switch (t) {
-    case at::kChar: return "torch.int8";
-    case at::kShort: return "torch.int16";
-    case at::kInt: return "torch.int32";
-    case at::kLong: return "torch.int64";
-    case at::kBool: return "torch.bool";
-    default: return c10::toString(t);
-  }
-}
+std::string dtype_name(at::ScalarType t) { return "torch." + c10::getDtypeNames(t).first; }
 
 int dt(at::ScalarType t) {
   switch (t) {
