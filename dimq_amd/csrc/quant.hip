@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void product_table_kernel(const void* __r
 struct CentreRow {
   float sv[256];  // centres in ascending order (ties by index)
   int si[256];    // their indices
-  __attribute__((aligned(16))) float raw[256];  // padded to a multiple of 4 with +inf
+  __attribute__((aligned(16))) float raw[256];  // WIDE: padded to a multiple of 4 with +inf
   int first_nan, first_pinf, first_ninf;  // first NaN / +inf / -inf centre, K if none
 };
 
@@ -89,13 +89,17 @@ __device__ __forceinline__ float centre_dist(float x, float c) {
 }
 
 // Whole work-group: the row's K (1..256) centres into `r`.
+// WIDE: the ranks from four centres per LDS read (4,096 x 4,096 weights, 64 and
+// 256 centres per row: 43.5 -> 42.1 and 84.6 -> 78.9 us; but 20,000 rows of 9,
+// where the set-up is most of the time, 29 -> 38 at 17 centres).
+template <bool WIDE>
 __device__ void centre_row_setup(const float* __restrict__ c, int K, CentreRow& r) {
   if (threadIdx.x == 0) {
     r.first_nan = K;
     r.first_pinf = K;
     r.first_ninf = K;
   }
-  const int K4 = (K + 3) & ~3;
+  const int K4 = WIDE ? (K + 3) & ~3 : K;
   for (int j = threadIdx.x; j < K4; j += blockDim.x) r.raw[j] = j < K ? c[j] : __builtin_inff();
   __syncthreads();
   for (int j = threadIdx.x; j < K; j += blockDim.x) {
@@ -105,10 +109,15 @@ __device__ void centre_row_setup(const float* __restrict__ c, int K, CentreRow& 
     if (v == -__builtin_inff()) atomicMin(&r.first_ninf, j);
     int rank = 0;
 #pragma unroll 8
-    for (int i = 0; i < K4; i += 4) {  // a padded entry is never below v, nor equal to it ahead of j
-      const float4 u = *reinterpret_cast<const float4*>(&r.raw[i]);
-      rank += ((u.x < v) || (u.x == v && i < j)) + ((u.y < v) || (u.y == v && i + 1 < j)) +
-              ((u.z < v) || (u.z == v && i + 2 < j)) + ((u.w < v) || (u.w == v && i + 3 < j));
+    for (int i = 0; i < K4; i += WIDE ? 4 : 1) {  // a padded entry is never below v, nor equal to it ahead of j
+      if constexpr (WIDE) {
+        const float4 u = *reinterpret_cast<const float4*>(&r.raw[i]);
+        rank += ((u.x < v) || (u.x == v && i < j)) + ((u.y < v) || (u.y == v && i + 1 < j)) +
+                ((u.z < v) || (u.z == v && i + 2 < j)) + ((u.w < v) || (u.w == v && i + 3 < j));
+      } else {
+        const float u = r.raw[i];
+        rank += (u < v) || (u == v && i < j);
+      }
     }
     // with a NaN centre ranks can collide; the sorted view is then unused
     r.sv[rank] = v;
@@ -212,6 +221,8 @@ __device__ __forceinline__ void store_some(uint8_t* __restrict__ idx, void* __re
 // 2^-19 for a < 2^19 g, two roundings of 2^-24 cannot close that, and with
 // 1e-18 < g and a < 1e18 no square under- or overflows.  Elements outside that
 // bound, NaN and infinite ones take the full scan.
+// KD = 0 (one element per thread): the sorted centres and, for every element,
+// the search and scan; the bound costs more to set up than it saves there.
 // 4,096 x 4,096 fp32 weights, 8 centres per row: 97.8 -> 29.5 us; 16:
 // 98.9 -> 33.1; 256: 129.1 -> 89.2; a plain copy of as many bytes 30.
 template <int KD, bool VEC, int E>
@@ -233,17 +244,27 @@ __global__ __launch_bounds__(kThreads) void nearest_centre_kernel(const void* __
   load_some<VEC, E>(w, dt, base, k, row_len, xn);  // before the centres are looked at
   bool fast = true;     // KD <= 8: every centre finite
   float limit = 0.0f;   // KD > 8: the bound above, 0 when the scan is always needed
-  float c[KD <= 8 ? KD : 1];
+  float c[KD > 0 && KD <= 8 ? KD : 1];
+  if constexpr (KD == 0) {
+    centre_row_setup<false>(cr, K, r);
+    for (int t = 0; t < trips && k < row_len; ++t, k += kTrip) {
+      if (t > 0) load_some<VEC, E>(w, dt, base, k, row_len, xn);
+      const int j[1] = {nearest_centre(xn[0], r, K)};
+      const float v[1] = {r.raw[j[0]]};
+      store_some<VEC, E>(idx, values, dt, base, k, row_len, j, v);
+    }
+    return;
+  }
   if constexpr (KD <= 8) {
 #pragma unroll
     for (int j = 0; j < KD; ++j) {
       c[j] = cr[j < K ? j : K - 1];
       fast &= __builtin_isfinite(c[j]);
     }
-    if (!fast) centre_row_setup(cr, K, r);
+    if (!fast) centre_row_setup<true>(cr, K, r);
   } else {
     if (threadIdx.x == 0) gap = __float_as_int(__builtin_inff());
-    centre_row_setup(cr, K, r);
+    centre_row_setup<true>(cr, K, r);
     bool fin = true;
     float mine = __builtin_inff();
     static_assert(KD <= kThreads, "one sorted centre per thread");
@@ -335,6 +356,7 @@ void launch_nearest_form(const void* w, int dt, int64_t row_len, const float* ce
                      centers, K, per_channel, idx, values, seg, trips)
   if (K <= 4) DIMQ_NEAREST(4);
   else if (K <= 8) DIMQ_NEAREST(8);
+  else if constexpr (E == 1) DIMQ_NEAREST(0);
   else if (K <= 16) DIMQ_NEAREST(16);
   else DIMQ_NEAREST(256);
 #undef DIMQ_NEAREST
@@ -345,9 +367,18 @@ int launch_nearest_centre(const void* w, int dt, int64_t rows, int64_t row_len, 
   if (rows == 0 || row_len == 0) return DIMQ_OK;
   const int pc = per_channel ? 1 : 0;
   const int64_t quads = (row_len + 4 * kThreads - 1) / (4 * kThreads);  // work-groups of a row at four elements a thread
-  if (rows * quads < device_cus()) {  // a small tensor: one element per thread, four times the work-groups
-    const int64_t seg = (row_len + kThreads - 1) / kThreads;
-    launch_nearest_form<false, 1>(w, dt, row_len, centers, K, pc, idx, values, seg, 1,
+  // One element per thread and trip: a small tensor (four times the
+  // work-groups), and short rows, where each work-group's time is the set-up
+  // (20,000 rows of 9: 9 centres 41 us on the four-element form, 19 here, 64
+  // centres 82 and 34; rows of 256 41 and 31, 64 and 47; of 300, 17 centres 51
+  // and 47; of 512 52 and 59; up to 8 centres, whose set-up is a load, rows of
+  // 9 30 and 22, of 256 28 and 31).
+  const int64_t one = K > 16 ? 352 : K > 8 ? kThreads : 64;
+  if (rows * quads < device_cus() || row_len <= one) {
+    const int trips = row_len <= one && row_len > kThreads && rows * quads >= device_cus() ? 2 : 1;
+    const int64_t seg = (row_len + kThreads * trips - 1) / (kThreads * trips);
+    DIMQ_CHECK(rows * seg < (int64_t)1 << 31, "tensor too large for one launch");
+    launch_nearest_form<false, 1>(w, dt, row_len, centers, K, pc, idx, values, seg, trips,
                                   static_cast<unsigned>(rows * seg), st);
     return check_launch("nearest centre");
   }

@@ -36,3 +36,19 @@ def test_nearest_centre_forms(gpu, K, rows, n, dt):
     off = torch.randn(n + 1, generator=g).to(dt).to(gpu)[1:]  # rows off the vector loads' alignment
     idx, val = ops.hard_quantize(off, cases[0][0].to(gpu), False)
     assert torch.equal(idx.cpu().long(), ((off.cpu().float()[:, None] - cases[0][0][None, :]) ** 2).argmin(1))
+
+
+@pytest.mark.parametrize("K", [8, 9, 16, 17, 64])
+@pytest.mark.parametrize("n", [9, 64, 65, 256, 257, 352, 353])
+def test_nearest_centre_row_lengths(gpu, K, n):
+    """More rows than CUs at the lengths where one element per thread gives way to four."""
+    from dimq_amd import ops
+    announce(f"nearest rows of {n} K={K}")
+    g = torch.Generator().manual_seed(K + n)
+    w, c = torch.randn(700, n, generator=g), torch.randn(700, K, generator=g)
+    c[1, 3] = c[1, 0]
+    w[0, :4] = torch.tensor([float("nan"), float("inf"), -1e30, 0.125])
+    idx, val = ops.hard_quantize(w.to(gpu), c.to(gpu), True)
+    want = ((w[:, :, None] - c[:, None, :]) ** 2).argmin(2)
+    assert torch.equal(idx.cpu().long(), want)
+    assert torch.equal(val.cpu(), torch.gather(c, 1, want))
