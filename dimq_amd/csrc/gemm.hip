@@ -32,12 +32,8 @@ int gemm_fast_tile(int tile, const GemmArgs& p, int bits) {
 }
 
 // Large-tile kernels (gemm_big.h) for Linear shapes with M > 64, K % 64 == 0
-// and aligned rows/streams.  The deep-pipeline tile (7, 64x128) is fastest
-// below 2,048 rows (128x128 tile against it at M 100, N = K = 4,096: 62 and 45
-// us; M 500: 61 and 41; M 1,024: 69 and 61; M 1,576, N 768, K 3,072: 47 and 31;
-// M 2,047, N 3,072, K 2,304: 53 and 49); the 2x2 128x128 tile (2) for long k
-// and fp32 activations above (M 12,608, K 3,072).  Returns -1 when the shape
-// does not qualify.
+// and aligned rows/streams: tile ids of launch_big_linear_modes, -1 when the
+// shape does not qualify.
 int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
   if (variant == DIMQ_VARIANT_SMALL_M || p.conv || !(bits == 2 || bits == 3 || bits == 4)) return -1;
   const int mode = epi_mode(p.epi);  // epilogues the large tiles are instantiated for
@@ -47,10 +43,24 @@ int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
   if (p.M <= 64 || p.K % 64 != 0 || !p.fast_b || !p.vec_a) return -1;
   // 256x256 shared-decode tiles for large M (measured on the ViT-B/16 shapes at
   // M 12,608, bf16: qkv 84 vs 104 us, proj 40 vs 50, fc1 114 vs 134, fc2 104 vs
-  // 133 against the best 128x128 tile); below M 2048 the 128x128 tiles fill
-  // the CUs better (M 1000: 17 vs 30 us).
-  if (p.M >= 2048 && x_dtype != DIMQ_F32) return 10;  // fp32 activations spill its registers
-  return p.M >= 2048 && p.K >= 2048 ? 2 : 7;
+  // 133 against the best 128x128 tile); fp32 activations spill its registers.
+  if (p.M >= 2048) return x_dtype != DIMQ_F32 ? 10 : p.K >= 2048 ? 2 : 7;
+  // Below 2,048 rows the deep-pipeline tile (7, 64x128) is faster than the
+  // 128x128 one (2) unless that one's work-groups fill their last round on the
+  // CUs (128x128 against 64x128 tiles: M 100, N = K = 4,096, 62 and 45 us; M
+  // 500 61 and 41; M 1,576, N 768, K 3,072 47 and 31).  There, 4-bit codebooks
+  // on fp16 and fp32 aside, its lower decode work per product wins: N 4,096, K
+  // 4,096, M 1,576 (416 tiles) bf16 3-bit 96 and 104 us, fp16 2-bit 73 and 81;
+  // M 2,047 (512) 104 and 118, 83 and 90; N 6,144, M 1,300 (528) 138 and 107,
+  // 1,800 (720) 151 and 165.  2-bit codes on 16-bit activations, the cheapest
+  // to decode, gain from a quarter of a round on (576 and 624 tiles 1.01 to
+  // 1.06 times as fast, the other types 0.85 to 1.0).
+  if (p.K >= 2048 && (bits < 4 || x_dtype == DIMQ_BF16)) {
+    const int64_t tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128), last = tiles % device_cus();
+    const bool half = x_dtype != DIMQ_F32;
+    if (last == 0 ? tiles > 400 || half : tiles > 400 && last > (bits == 2 && half ? 48 : 150)) return 2;
+  }
+  return 7;
 }
 
 // Whether the general pre-laid path (gemm_gen.hip) takes a Linear that no path

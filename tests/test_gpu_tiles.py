@@ -1,0 +1,41 @@
+"""Linears of 65 to 2,047 rows on either side of the rule that picks the 128x128 tile over the 64x128 one, against the
+dequantized product in float64.
+
+Bar: fp16 operands and fp32 sums, 2e-3 of the largest value plus the output's own rounding (conftest.out_tol, the bar
+of every weight-only kernel)."""
+
+import pytest
+import torch
+
+from tests.conftest import announce, out_tol
+from tests.test_gpu_general import _act, _close, _gen, _weights
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K, bits, x dtype, out dtype, activation, residual): 407 tiles of 128x128 and up, then 396 and 11 * 48 (their
+# last round is short), 4-bit fp16 (the other tile at any count)
+LINEAR = [
+    (1300, 4700, 2048, 2, "float16", "float16", None, False),
+    (1281, 4609, 2112, 3, "bfloat16", "float32", "relu", False),     # row and column tails, odd pitch
+    (1300, 4700, 2048, 4, "bfloat16", "bfloat16", None, True),
+    (1300, 4700, 2048, 3, "float32", "float16", "gelu", False),
+    (1300, 4600, 2048, 2, "float16", "float16", None, True),
+    (1300, 6100, 2048, 3, "bfloat16", "bfloat16", None, False),
+    (1300, 4700, 2048, 4, "float16", "float16", "relu", False),
+    (1100, 8100, 2048, 2, "bfloat16", "bfloat16", None, False),      # 576 tiles: 2-bit only
+    (1100, 8100, 2048, 3, "bfloat16", "bfloat16", None, False),
+]
+
+
+@pytest.mark.parametrize("M,N,K,bits,xdt,ydt,act,res", LINEAR)
+def test_tile_choice_below_2048_rows(gpu, M, N, K, bits, xdt, ydt, act, res):
+    from dimq_amd import ops
+    announce(f"tiles {M} {N} {K} {bits} {xdt}")
+    xdt, ydt = getattr(torch, xdt), getattr(torch, ydt)
+    g = _gen(M + N + bits)
+    packed, cb, w = _weights(N, K, bits, True, g)
+    x, bias = torch.randn(M, K, generator=g).to(xdt), torch.randn(N, generator=g)
+    r = torch.randn(M, N, generator=g).to(ydt) if res else None
+    y = ops.dimq_linear_codebook(x.to(gpu), packed.to(gpu), cb.to(gpu), bits, bias.to(gpu), N, K, out_dtype=ydt,
+                                 residual=None if r is None else r.to(gpu), activation=act)
+    _close(y, _act(x.double() @ w.T + bias.double(), r, act), out_tol(ydt))
