@@ -67,14 +67,22 @@ int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
 // with a workspace of its own does: every shape beyond the decode shapes that
 // the large tiles' k steps or codebooks do not fit.  At 16 < M <= 64 with
 // K % 128 == 0 the register-codebook tiles decode each weight once or twice
-// only, and win while K is short (M 17, K 384, N 3,072: 11.7 against 12.2 us;
-// M 32, K 3,072, N 768: 30.4 against 16.8).
-// And while the weights are few: laying out 16.8 M of them takes 25 us (M 20,
-// K = N = 4,096: 38.8 against 43.1).
-bool gen_wants_linear(int64_t M, int64_t K, int64_t N, int bits) {
+// only, in a time that hardly depends on N, while laying the weights out grows
+// with N.  The general path wins while K is long and N small, up to 2,048
+// outputs (2-bit codes, which decode faster, 1,536), from 49 rows on half as
+// many more: K 2,048, 4-bit, M 17, N 2,048 22.4 against 20.4 us, N 3,072 22.5
+// and 24.8, N 4,096 22.5 and 29.8; M 64, N 3,072 27.0 and 25.3; 2-bit, K 1,536,
+// M 17, N 1,536 15.7 and 15.6, N 2,048 15.7 and 16.5; M 32, K 3,072, N 768 31.1
+// and 16.8; M 17, K 384, N 3,072 11.7 and 12.2.  W4A4 (a4), whose tiles need
+// the activations quantized first: up to 3,072 (K 2,048, M 17, N 3,072 24.0 and
+// 23.5, N 4,096 24.2 and 28.4).
+bool gen_wants_linear(int64_t M, int64_t K, int64_t N, int bits, bool a4 = false) {
   if (M <= 16) return false;
   if (bits == 8 || K % 64 != 0) return true;
-  return M <= 64 && (K % 128 != 0 || (K >= 1024 && N * K <= (8ll << 20)));
+  if (M > 64) return false;
+  if (K % 128 != 0) return true;
+  const int64_t most = a4 ? 3072 : bits == 2 ? (M > 48 ? 2048 : 1536) : (M > 48 ? 3072 : 2048);
+  return K >= 1024 && N <= most && N * K <= (8ll << 20);
 }
 
 // k ranges of a Linear on the 64x128 tiles.  A 64-k stage takes 0.45 us there.
@@ -431,7 +439,7 @@ extern "C" int64_t dimq_linear_lut_workspace_bytes(int64_t M, int64_t in_feature
 // where that path runs: codebooks that are not fp16, and in_features off the
 // fast tiles' k steps.
 static bool lut_wants_gen(int64_t M, int64_t in_features, int64_t out_features, int cb_dtype) {
-  return cb_dtype != DIMQ_F16 || gen_wants_linear(M, in_features, out_features, 4);
+  return cb_dtype != DIMQ_F16 || gen_wants_linear(M, in_features, out_features, 4, true);
 }
 
 extern "C" int64_t dimq_linear_lut_full_workspace_bytes(int x_dtype, int64_t M, int64_t out_features,

@@ -37,3 +37,23 @@ def test_general_path_workspace_is_bounded():
     assert 0 < lin(20_000_000, 3, 16, 4, _C.F32) <= limit + weights
     # one image beyond the bound goes by itself
     assert limit < _conv_ws(_C.F32, _C.NCHW, 2, 64, 640, 640, 64, 3, 64) <= 640 * 640 * 64 * 20 + weights
+
+
+@pytest.mark.parametrize("M,K,N,bits,general", [
+    (17, 2048, 2048, 4, True), (17, 2048, 3072, 4, False), (17, 1024, 8192, 4, False), (48, 2048, 4096, 3, False),
+    (64, 2048, 3072, 4, True), (64, 2048, 3200, 4, False), (64, 1024, 4096, 4, False),
+    (17, 1536, 1536, 2, True), (17, 1536, 2048, 2, False), (49, 1536, 2048, 2, True), (64, 1024, 8192, 2, False),
+    (17, 384, 3072, 4, False), (32, 3072, 768, 4, True), (17, 8192, 1024, 4, True), (64, 2112, 8192, 4, True),
+    (17, 4096, 4096, 8, True), (17, 1000, 4096, 4, True), (16, 1000, 4096, 8, False)])
+def test_general_path_on_few_rows(M, K, N, bits, general):
+    """Up to 64 rows with K % 128 == 0 the general path takes only the layers of few outputs: laying the weights of wider
+    ones out costs more than the register-codebook tiles take."""
+    from dimq_amd import _C
+    need = _C.lib.dimq_linear_codebook_full_workspace_bytes(M, K, N, bits, _C.BF16)
+    assert (need >= N * K * 2) == general
+
+
+@pytest.mark.parametrize("M,K,N,general", [(17, 2048, 3072, True), (17, 2048, 3200, False), (64, 1024, 8192, False)])
+def test_general_path_on_few_w4a4_rows(M, K, N, general):
+    from dimq_amd import _C
+    assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F16) >= N * K * 2) == general
