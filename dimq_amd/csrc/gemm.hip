@@ -435,13 +435,24 @@ extern "C" int64_t dimq_linear_lut_workspace_bytes(int64_t M, int64_t in_feature
   return (M * in_features * 2 + 255) / 256 * 256;
 }
 
-// dimq_linear_lut_workspace_bytes, or what the general pre-laid path needs
-// where that path runs: codebooks that are not fp16, and in_features off the
-// fast tiles' k steps.
+// Whether the general pre-laid path takes a W4A4 Linear: in_features off the
+// fast tiles' k steps, few rows, and codebooks that are not fp16 -- unless
+// their generic A4 tiles (64x128, K % 128 == 0) fill the chip.  Those take per
+// k about 28 ns in up to one tile per CU, 36 in up to two, then 66 per 1,024;
+// the general path 1.65 ns per 1,000 outputs to lay hi and lo planes out and 8
+// per million products of M * N.  4,096 x 4,096: M 1 to 16 107 against 42 us,
+// M 512 115 and 94, M 1,024 149 and 168, M 4,096 555 and 640; 8,192 x 8,192:
+// M 16 211 and 147, M 512 281 and 362; K 1,024, N 4,096, M 4,096 179 and 164.
 static bool lut_wants_gen(int64_t M, int64_t in_features, int64_t out_features, int cb_dtype) {
-  return cb_dtype != DIMQ_F16 || gen_wants_linear(M, in_features, out_features, 4, true);
+  if (cb_dtype == DIMQ_F16) return gen_wants_linear(M, in_features, out_features, 4, true);
+  if (in_features % kKM != 0 || in_features <= 2048) return true;
+  const int64_t tiles = ((M + 63) / 64) * ((out_features + 127) / 128);
+  const double a4 = tiles <= device_cus() ? 28.0 : tiles <= 2 * device_cus() ? 36.0 : 0.0645 * tiles;
+  return 1.65e-3 * out_features + 8e-6 * M * out_features < a4;
 }
 
+// dimq_linear_lut_workspace_bytes, or what the general pre-laid path needs
+// where it runs.
 extern "C" int64_t dimq_linear_lut_full_workspace_bytes(int x_dtype, int64_t M, int64_t out_features,
                                                         int64_t in_features, int cb_dtype) {
   const int64_t small = dimq_linear_lut_workspace_bytes(M, in_features, cb_dtype);

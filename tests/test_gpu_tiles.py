@@ -7,6 +7,7 @@ of every weight-only kernel)."""
 import pytest
 import torch
 
+import oracle
 from tests.conftest import announce, out_tol
 from tests.test_gpu_general import _act, _close, _gen, _weights
 
@@ -39,3 +40,17 @@ def test_tile_choice_below_2048_rows(gpu, M, N, K, bits, xdt, ydt, act, res):
     y = ops.dimq_linear_codebook(x.to(gpu), packed.to(gpu), cb.to(gpu), bits, bias.to(gpu), N, K, out_dtype=ydt,
                                  residual=None if r is None else r.to(gpu), activation=act)
     _close(y, _act(x.double() @ w.T + bias.double(), r, act), out_tol(ydt))
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 8192, 2176), (517, 8200, 2304)])
+@pytest.mark.parametrize("cdt,xdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.float16)])
+def test_w4a4_products_that_fill_the_chip(gpu, M, N, K, cdt, xdt):
+    """Codebooks that are not fp16 on the generic A4 tiles: exact codes and hi + lo planes, 2e-6 of the largest value."""
+    from dimq_amd import ops
+    announce(f"w4a4 tiles {M} {N} {K} {cdt} {xdt}")
+    g = _gen(N)
+    packed, cb, w = _weights(N, K, 4, False, g, cdt)
+    x, bias = torch.randn(M, K, generator=g).to(xdt), torch.randn(N, generator=g)
+    y = ops.dimq_linear_lut(x.to(gpu), packed.to(gpu), cb.to(gpu), 0.2371, 7, bias.to(gpu), N, K)
+    a = torch.from_numpy(oracle.quantize_act_u4(x.float(), 0.2371, 7)).double() - 7
+    _close(y, 0.2371 * (a @ w.T) + bias.double(), 2e-6)

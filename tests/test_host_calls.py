@@ -57,3 +57,13 @@ def test_general_path_on_few_rows(M, K, N, bits, general):
 def test_general_path_on_few_w4a4_rows(M, K, N, general):
     from dimq_amd import _C
     assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F16) >= N * K * 2) == general
+
+
+@pytest.mark.parametrize("M,K,N,general", [
+    (1, 4096, 4096, True), (16, 8192, 8192, True), (128, 8192, 8192, True), (512, 8192, 8192, False),
+    (512, 4096, 4096, True), (768, 4096, 4096, True), (1024, 4096, 4096, False), (4096, 4096, 4096, False),
+    (4096, 1024, 4096, True), (4096, 3072, 768, True), (4096, 4000, 4096, True)])
+def test_general_path_on_w4a4_codebooks_that_are_not_fp16(M, K, N, general):
+    """Their generic tiles keep the products that fill the chip."""
+    from dimq_amd import _C
+    assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F32) >= N * K * 4) == general
