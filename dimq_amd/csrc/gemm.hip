@@ -76,9 +76,20 @@ int gemm_big_tile(const GemmArgs& p, int bits, int x_dtype, int variant) {
 // and 16.8; M 17, K 384, N 3,072 11.7 and 12.2.  W4A4 (a4), whose tiles need
 // the activations quantized first: up to 3,072 (K 2,048, M 17, N 3,072 24.0 and
 // 23.5, N 4,096 24.2 and 28.4).
+// K % 32 == 0 off the large tiles' 64-k steps: the register-codebook tiles'
+// 64x128 form, taken below 256 tiles of 128x256, is faster once its tiles fill
+// the chip: per k about 23 ns against 0.9 per 1,000 outputs of layout and 4.5
+// per million products of M * N here, which is N (M + 200) about 4.8M (W4A4,
+// whose activations are quantized first: 5.5M).  N 4,096, K 4,000, M 500 91
+// against 57 us, M 1,500 103 and 130, M 2,047 (the other form) 339 and 167; N
+// 8,192, K 8,160, M 500 158 and 189.
 bool gen_wants_linear(int64_t M, int64_t K, int64_t N, int bits, bool a4 = false) {
   if (M <= 16) return false;
-  if (bits == 8 || K % 64 != 0) return true;
+  if (bits == 8) return true;
+  if (K % 64 != 0) {
+    const bool filled = K % 32 == 0 && K >= 960 && N * (M + 200) > (a4 ? 5500000 : 4800000);
+    return !(filled && ((M + 127) / 128) * ((N + 255) / 256) < kCUs);
+  }
   if (M > 64) return false;
   if (K % 128 != 0) return true;
   const int64_t most = a4 ? 3072 : bits == 2 ? (M > 48 ? 2048 : 1536) : (M > 48 ? 3072 : 2048);

@@ -25,6 +25,8 @@ LINEAR = [
     (1300, 4700, 2048, 4, "float16", "float16", "relu", False),
     (1100, 8100, 2048, 2, "bfloat16", "bfloat16", None, False),      # 576 tiles: 2-bit only
     (1100, 8100, 2048, 3, "bfloat16", "bfloat16", None, False),
+    (1500, 4096, 992, 4, "float16", "float16", None, False),         # K % 32 == 0: the 64x128 register-codebook tiles
+    (1501, 4100, 992, 3, "float32", "bfloat16", "relu", True),
 ]
 
 

@@ -67,3 +67,13 @@ def test_general_path_on_w4a4_codebooks_that_are_not_fp16(M, K, N, general):
     """Their generic tiles keep the products that fill the chip."""
     from dimq_amd import _C
     assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F32) >= N * K * 4) == general
+
+
+@pytest.mark.parametrize("M,K,N,general", [
+    (500, 4000, 4096, True), (1500, 4000, 4096, False), (2047, 4000, 4096, True), (500, 8160, 8192, False),
+    (1000, 8160, 8192, True), (1500, 4001, 4096, True), (1500, 928, 4096, True), (2047, 4000, 2048, True)])
+def test_general_path_off_the_large_tiles_k_steps(M, K, N, general):
+    """K % 32 == 0: the register-codebook tiles keep the products that fill the chip on their smaller form."""
+    from dimq_amd import _C
+    assert (_C.lib.dimq_linear_codebook_full_workspace_bytes(M, K, N, 4, _C.F16) >= N * K * 2) == general
+    assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F16) >= N * K * 2) == general
