@@ -185,25 +185,28 @@ int linear_codebook_impl(const void* x, int x_dtype, int64_t M, int64_t K, int64
     if (rc >= 0) return rc;
   }
   const int big = gemm_big_tile(p, bits, x_dtype, variant);
-  if (big < 0 && M > 16 && (M > 64 || gen_wants_linear(M, K, N, bits)) && workspace != nullptr &&
-      aligned(workspace, 256) && variant != DIMQ_VARIANT_SMALL_M) {
-    const GenPlan g = gen_plan(p, bits, x_dtype, false, aligned(x, 16));
-    if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, bits, x_dtype, workspace, s);
-  }
-  if (big >= 0 && workspace != nullptr && aligned(workspace, 256)) {
-    const int sp = big_linear_splits(M, K, N, big);
+  if (workspace != nullptr && aligned(workspace, 256)) {
+    // the first pass of split k has no epilogue: any may follow in the second
+    GemmArgs plain = p;
+    plain.epi = Epi{};
+    const int tile = gemm_big_tile(plain, bits, x_dtype, variant);
+    const int sp = tile >= 0 ? big_linear_splits(M, K, N, tile) : 1;
     if (sp > 1 && workspace_bytes >= split_bytes(sp, M, ldy)) {
       const GemmArgs q = split_args(p, sp, workspace);
       int rc = DIMQ_OK;
       switch (bits) {
-        case 2: rc = launch_big_b2(q, x_dtype, big, s); break;
-        case 3: rc = launch_big_b3(q, x_dtype, big, s); break;
-        default: rc = launch_big_b4(q, x_dtype, big, s); break;
+        case 2: rc = launch_big_b2(q, x_dtype, tile, s); break;
+        case 3: rc = launch_big_b3(q, x_dtype, tile, s); break;
+        default: rc = launch_big_b4(q, x_dtype, tile, s); break;
       }
       if (rc != DIMQ_OK) return rc;
       launch_split_reduce(p, static_cast<const float*>(workspace), sp, nullptr, x_dtype, bits, x_dtype != DIMQ_F16,
                           false, s);
       return check_launch("linear_codebook (split k)");
+    }
+    if (big < 0 && gen_wants_linear(M, K, N, bits) && variant != DIMQ_VARIANT_SMALL_M) {
+      const GenPlan g = gen_plan(p, bits, x_dtype, false, aligned(x, 16));
+      if (g.ok && workspace_bytes >= g.bytes) return launch_gen(p, g, bits, x_dtype, workspace, s);
     }
   }
   if (big >= 0) {

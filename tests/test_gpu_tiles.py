@@ -56,3 +56,20 @@ def test_w4a4_products_that_fill_the_chip(gpu, M, N, K, cdt, xdt):
     y = ops.dimq_linear_lut(x.to(gpu), packed.to(gpu), cb.to(gpu), 0.2371, 7, bias.to(gpu), N, K)
     a = torch.from_numpy(oracle.quantize_act_u4(x.float(), 0.2371, 7)).double() - 7
     _close(y, 0.2371 * (a @ w.T) + bias.double(), 2e-6)
+
+
+@pytest.mark.parametrize("M,K", [(130, 768), (130, 3072), (1000, 768), (1000, 3072), (300, 2112)])
+@pytest.mark.parametrize("act,xdt,ydt", [("relu", "float16", "float16"), ("gelu", "bfloat16", "float32")])
+def test_epilogues_the_large_tiles_lack(gpu, M, K, act, xdt, ydt):
+    """Residual and activation together: k split where the same layer without them splits it, the generic tiles where
+    not; a workspace from the size query is then used by neither or by both."""
+    from dimq_amd import ops
+    announce(f"residual + {act} {M} {K} {xdt}")
+    N = 768
+    xdt, ydt = getattr(torch, xdt), getattr(torch, ydt)
+    g = _gen(M + K)
+    packed, cb, w = _weights(N, K, 4, True, g)
+    x, bias, r = torch.randn(M, K, generator=g).to(xdt), torch.randn(N, generator=g), torch.randn(M, N, generator=g).to(ydt)
+    y = ops.dimq_linear_codebook(x.to(gpu), packed.to(gpu), cb.to(gpu), 4, bias.to(gpu), N, K, out_dtype=ydt,
+                                 residual=r.to(gpu), activation=act)
+    _close(y, _act(x.double() @ w.T + bias.double(), r, act), out_tol(ydt))
