@@ -745,6 +745,8 @@ GenPlan gen_plan(const GemmArgs& p, int bits, int x_dtype, bool a4, bool in_plac
   // 32-bit pixel offsets and row numbers in the kernel
   if (g.pixels * xpitch >= (1ll << 31) || p.M >= (1ll << 31) - 256 || p.N >= (1ll << 31) - 256) return g;
   if (g.conv && (p.cH * p.cW >= (1ll << 31) || taps * g.cg >= (1ll << 30))) return g;
+  // a launch dimension holds fewer than 2^32 threads; the tiles without a workspace are larger
+  if (cdiv(p.M, kGenB) * cdiv(p.N, kGenB) >= (1ll << 24)) return g;
   const int64_t rows = groups * p.N, ldw = g.kp * (g.hilo ? 2 : 1), nk = ldw / kGenK;
   const int64_t cpl = cdiv(g.cg, kGenChan);
   const bool guard = !a4 && (x_dtype == DIMQ_F32 || x_dtype == DIMQ_BF16);

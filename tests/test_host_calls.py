@@ -77,3 +77,11 @@ def test_general_path_off_the_large_tiles_k_steps(M, K, N, general):
     from dimq_amd import _C
     assert (_C.lib.dimq_linear_codebook_full_workspace_bytes(M, K, N, 4, _C.F16) >= N * K * 2) == general
     assert (_C.lib.dimq_linear_lut_full_workspace_bytes(_C.F32, M, N, K, _C.F16) >= N * K * 2) == general
+
+
+def test_general_path_leaves_products_beyond_one_launch():
+    """2^24 work-groups of 256 threads exceed a launch dimension: those calls keep the larger tiles."""
+    from dimq_amd import _C
+    lin = _C.lib.dimq_linear_codebook_full_workspace_bytes
+    assert lin(4 << 20, 448, 16384, 8, _C.F16) == 0
+    assert lin(4 << 20, 448, 16320, 8, _C.F16) > 0
