@@ -258,11 +258,13 @@ def _model_workload(name, workload, dev, rotations, qmodel, xs_cpu, flops_per_im
     def step(i):
         return qmodel(xs[i])
 
+    cpu = []  # this workload's model, built when first asked for
+
     def cpu_model():
         import oracle
-        if "cpu" not in _model_workload.cache:
-            _model_workload.cache["cpu"] = oracle.dequantized_model(qmodel)
-        return _model_workload.cache["cpu"]
+        if not cpu:
+            cpu.append(oracle.dequantized_model(qmodel))
+        return cpu[0]
 
     @torch.no_grad()
     def cpu_step(sample):
@@ -282,9 +284,6 @@ def _model_workload(name, workload, dev, rotations, qmodel, xs_cpu, flops_per_im
         check=check, extra_config={"global_batch": batch, **extra},
         per_set_bytes=xs_cpu.numel() * 2,
     )
-
-
-_model_workload.cache = {}
 
 
 def make_vit(dev, rotations):
