@@ -43,11 +43,12 @@ LINEAR = [
     (17, 33, 33, 3, "float16", "float16", True, None, False),        # every size off its tile; one k stage and a bit
     (31, 70, 749, 4, "float32", "float32", False, "relu", True),     # split k, rows converted
     (64, 536, 3183, 4, "float16", "bfloat16", True, "gelu", False),  # odd K: fp16 rows copied to the padded pitch
-    (65, 64, 96, 8, "float16", "float32", True, None, False),        # K % 32 == 0: rows read in place
+    (65, 64, 96, 8, "float16", "float32", True, None, False),        # K off the 64-k stages: rows copied
+    (65, 64, 192, 8, "float16", "float32", True, None, False),       # K % 64 == 0: rows read in place
     (130, 257, 1000, 8, "bfloat16", "bfloat16", False, None, True),
     (300, 200, 150, 2, "bfloat16", "float16", True, "relu", True),
-    (4133, 1100, 91, 4, "float32", "float16", True, None, False),    # 128 x 128 tiles, odd pitch
-    (33000, 40, 65, 3, "float16", "float16", True, None, True),      # 128 x 64 tiles
+    (4133, 1100, 91, 4, "float32", "float16", True, None, False),    # many tiles each way, odd pitch
+    (33000, 40, 65, 3, "float16", "float16", True, None, True),      # one column of many tiles
 ]
 
 
@@ -74,8 +75,8 @@ CONV = [
     (5, 24, 19, 15, 64, 5, 5, 1, 2, 1, 1, 8, "float16", "float16", True, "gelu", False),   # read in place
     (4, 256, 14, 14, 96, 3, 3, 1, 1, 1, 1, 2, "float16", "float32", False, None, False),   # split k
     (2, 128, 9, 9, 72, 1, 1, 2, 0, 1, 2, 4, "float16", "bfloat16", True, None, False),     # groups, in place
-    (17, 65, 60, 33, 140, 3, 3, 1, 1, 1, 1, 4, "float16", "float16", False, "relu", False),  # 128 x 128 tiles
-    (40, 16, 40, 41, 8, 3, 3, 1, 1, 1, 1, 3, "bfloat16", "bfloat16", False, None, False),  # 128 x 64 tiles
+    (17, 65, 60, 33, 140, 3, 3, 1, 1, 1, 1, 4, "float16", "float16", False, "relu", False),  # many tiles each way
+    (40, 16, 40, 41, 8, 3, 3, 1, 1, 1, 1, 3, "bfloat16", "bfloat16", False, None, False),  # one column of many tiles
     (1, 8, 5, 5, 16, 7, 7, 1, 3, 1, 1, 4, "float32", "float16", True, None, False),        # taps mostly outside
 ]
 

@@ -1,6 +1,6 @@
 """Nearest-centre assignment: the register form (up to 8 centres) and the sorted form (16, 256) at the counts where
-one gives way to the next, aligned and unaligned rows, several trips per work-group, and centres whose gaps force the
-full scan; exact against torch's argmin."""
+one gives way to the next, aligned and unaligned rows, one, two and four trips per work-group, and centres whose gaps
+force the full scan; exact against torch's argmin (the first of equal distances)."""
 
 import pytest
 import torch
@@ -52,3 +52,27 @@ def test_nearest_centre_row_lengths(gpu, K, n):
     want = ((w[:, :, None] - c[:, None, :]) ** 2).argmin(2)
     assert torch.equal(idx.cpu().long(), want)
     assert torch.equal(val.cpu(), torch.gather(c, 1, want))
+
+
+@pytest.mark.parametrize("K", [8, 16, 256])
+@pytest.mark.parametrize("rows,n", [(4096, 1028), (4100, 1025),   # two trips of 1,024, the second nearly empty
+                                    (2100, 4100), (2100, 4099),   # four, the second work-group of a row with one
+                                    (1, 5_000_003), (1, 5_000_004)])
+def test_nearest_centre_several_trips(gpu, K, rows, n):
+    from dimq_amd import ops
+    announce(f"nearest trips K={K} rows={rows} n={n}")
+    g = torch.Generator().manual_seed(K + rows + n)
+    w, c = torch.randn(rows, n, generator=g).to(gpu), torch.randn(rows, K, generator=g).to(gpu)
+    w[:, -1] = float("nan")  # the last element of the ragged trip: index 0
+    idx, val = ops.hard_quantize(w, c, True)
+    order = torch.arange(K, device=gpu, dtype=torch.int16)
+    per = max(1, 4_000_000 // K // n)
+    for r in range(0, rows, per):
+        for k in range(0, n, 2_000_000 // K * 8):
+            ws, cs = w[r:r + per, k:k + 2_000_000 // K * 8], c[r:r + per]
+            d = (ws[:, :, None] - cs[:, None, :]) ** 2
+            want = torch.where(d == d.amin(2, keepdim=True), order, torch.tensor(K, dtype=torch.int16, device=gpu)).amin(2)
+            want[want == K] = 0  # a NaN equals nothing
+            got = idx[r:r + per, k:k + ws.shape[1]]
+            assert torch.equal(got.short(), want)
+            assert torch.equal(val[r:r + per, k:k + ws.shape[1]], torch.gather(cs, 1, want.long()))

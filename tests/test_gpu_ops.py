@@ -172,7 +172,7 @@ def test_hard_quantize_ties_and_specials(gpu, K):
         bad = (idx.cpu().long() != want).nonzero().flatten()
         assert bad.numel() == 0, [(float(w[i]), int(idx[i]), int(want[i])) for i in bad[:5]]
         assert np.array_equal(idx.cpu().numpy(), oracle.hard_quantize(w, cc)[0])
-    big = torch.randn(3, 1 << 20, generator=g)   # 4096+ segments: 16 elements per thread
+    big = torch.randn(3, 1 << 20, generator=g)   # 3,072 work-groups of four elements per thread
     cb = torch.randn(3, K, generator=g)
     idx, val = ops.hard_quantize(big.to(gpu), cb.to(gpu), True)
     for r in range(3):

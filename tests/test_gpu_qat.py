@@ -163,8 +163,8 @@ def test_qat_deterministic_and_errors(gpu):
 @pytest.mark.parametrize("tau", [1e-1, 1e-4])
 def test_qat_centre_counts_and_chunk_edges(gpu, n, K, tau):
     """The register instances (4, 8, 16 centres) at counts below their size, the LDS instance at centre tiles that
-    end early, element counts next to a chunk's edge, and more chunks than work-groups (2,200,003 weights); both
-    functions and the separation loss in one backward."""
+    end early, element counts next to a chunk's edge, and more chunks than the work-groups of a backward of up to 16
+    centres (2,200,003 weights); both functions and the separation loss in one backward."""
     from dimq_amd import qat
     announce(f"qat edges n={n} K={K} tau={tau}")
     w, c = _case(n, K, 5 * n + K)

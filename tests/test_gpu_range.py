@@ -60,10 +60,10 @@ LINEAR_CASES = [
     ("gemv_direct_k1024", 5, 64, 1024, 2),
     ("gemv_cb", 5, 77, 1000, 3),
     ("gemm_fast", 40, 256, 512, 4),
-    ("gemm_cb", 40, 100, 100, 2),
-    ("gemm_cb8", 40, 64, 256, 8),
-    ("deep_128x128", 200, 256, 768, 4),
-    ("big_128x128", 130, 200, 2048, 3),
+    ("general_k_off_steps", 40, 100, 100, 2),
+    ("general_8bit", 40, 64, 256, 8),
+    ("deep_64x128", 200, 256, 768, 4),
+    ("split_k_64x128", 130, 200, 2048, 3),
     # M >= 2048: activations converted to fp16 in the pre-decode launch, per-row flags, one tile shape each
     ("predecoded_128x128", 2100, 300, 192, 4),
     ("predecoded_128x384", 2200, 768, 64, 3),
@@ -143,8 +143,8 @@ def test_linear_codebook_range_inf_nan_inputs(gpu, M):
 CONV_CASES = [
     # id, B, C, H, W, OC, KH, stride, pad, bits, layout, prepared
     ("implicit_gemm_nhwc", 2, 64, 12, 12, 64, 3, 1, 1, 2, "nhwc", True),
-    ("generic_nchw", 2, 16, 10, 9, 32, 3, 1, 1, 3, "nchw", False),
-    ("generic_stem", 2, 3, 31, 29, 16, 7, 2, 3, 8, "nchw", False),
+    ("general_nchw", 2, 16, 10, 9, 32, 3, 1, 1, 3, "nchw", False),
+    ("general_stem", 2, 3, 31, 29, 16, 7, 2, 3, 8, "nchw", False),
 ]
 
 
