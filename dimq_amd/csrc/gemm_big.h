@@ -1239,11 +1239,12 @@ int launch_big_conv_bits(const GemmArgs& p, int xt, int tile, hipStream_t s) {
 }
 
 // Linear tile ids (WGM x WGN waves of (MBLK*32) x (NBLK*32)):
-//   2: 128x128 (2x2, 64x64)   7: 64x128 deep pipeline (kDeepMblk)
+//   2: 128x128 (2x2, 64x64), not for 4-bit codes on fp16 (gemm_big_tile)
+//   7: 64x128 deep pipeline (kDeepMblk)
 //  10: 256x256 shared decode (4x2, 64x128), next stage's decode woven between the MFMAs
 // Epilogue modes: none / relu / gelu / residual on each; for fp16 inputs (the
-// W4A4 activation codes) also none / relu / gelu with the next layer's
-// activation quantization.
+// W4A4 activation codes) on tiles 7 and 10 also none / relu / gelu with the
+// next layer's activation quantization.
 template <int BITS, int XT>
 int launch_big_linear_modes(const GemmArgs& p, int tile, int mode, hipStream_t s) {
   if (p.splits > 1) return launch_big_split<BITS, XT, 1, 4, 2, 1, false>(p, s);
@@ -1253,8 +1254,7 @@ int launch_big_linear_modes(const GemmArgs& p, int tile, int mode, hipStream_t s
 #define DIMQ_QMODE(M)                                                                \
   case M:                                                                            \
     if (tile == 10) return launch_lds<BITS, XT, 4, 2, 2, 4, M, 8>(p, s);             \
-    if (tile == 7) return launch_deep<BITS, XT, kDeepMblk, M>(p, s);                         \
-    return launch_big<BITS, XT, 2, 2, 2, 2, false, M>(p, s);
+    return launch_deep<BITS, XT, kDeepMblk, M>(p, s);
         DIMQ_QMODE(kEpiQuant)
         DIMQ_QMODE(kEpiRelu | kEpiQuant)
         DIMQ_QMODE(kEpiGelu | kEpiQuant)
@@ -1270,7 +1270,8 @@ int launch_big_linear_modes(const GemmArgs& p, int tile, int mode, hipStream_t s
       default: return launch_lds<BITS, XT, 4, 2, 2, 4, kEpiNone, 8>(p, s);
     }
   }
-  if (tile == 7) {
+  constexpr bool kBig = !(XT == DIMQ_F16 && BITS == 4);
+  if (!kBig || tile == 7) {
     switch (mode) {
       case kEpiRelu: return launch_deep<BITS, XT, kDeepMblk, kEpiRelu>(p, s);
       case kEpiGelu: return launch_deep<BITS, XT, kDeepMblk, kEpiGelu>(p, s);
@@ -1278,11 +1279,13 @@ int launch_big_linear_modes(const GemmArgs& p, int tile, int mode, hipStream_t s
       default: return launch_deep<BITS, XT, kDeepMblk, kEpiNone>(p, s);
     }
   }
-  switch (mode) {
-    case kEpiRelu: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiRelu>(p, s);
-    case kEpiGelu: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiGelu>(p, s);
-    case kEpiRes: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiRes>(p, s);
-    default: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiNone>(p, s);
+  if constexpr (kBig) {
+    switch (mode) {
+      case kEpiRelu: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiRelu>(p, s);
+      case kEpiGelu: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiGelu>(p, s);
+      case kEpiRes: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiRes>(p, s);
+      default: return launch_big<BITS, XT, 2, 2, 2, 2, false, kEpiNone>(p, s);
+    }
   }
 }
 
