@@ -140,9 +140,9 @@ Tensor linear_lut(const Tensor& x, const Tensor& packed_w, const Tensor& codeboo
   const Bias b(bias, out_features, "out_features");
   const int64_t M = xc.numel() / in_features;
   const Tensor y = at::empty(out_shape(x, out_features), x.options().dtype(at::kFloat));
+  const On on(xc);
   const Tensor ws = spare_workspace(
       dimq_linear_lut_full_workspace_bytes(dt(xc), M, out_features, in_features, dt(cb)), xc);
-  const On on(xc);
   check_rc(dimq_linear_lut_ws(ptr(xc), dt(xc), M, u8(pw), pw.numel(), ptr(cb), dt(cb), cb.numel(), act_scale, act_zp,
                               b.p, b.dtype, b.n, out_features, in_features, static_cast<float*>(y.data_ptr()), ptr(ws),
                               ws.defined() ? ws.numel() : 0, on.stream));
@@ -165,12 +165,12 @@ Tensor conv2d_lut(const Tensor& x, const Tensor& packed_w, const Tensor& codeboo
   const Bias b(bias, out_channels, "out_channels");
   const Tensor y = at::empty({B, out_channels, conv_out(H, pad_h, dilation_h, kernel_h, stride_h),
                               conv_out(W, pad_w, dilation_w, kernel_w, stride_w)}, x.options().dtype(at::kFloat));
+  const On on(xc);
   Tensor ws;
   if (y.numel() > 0)
     ws = spare_workspace(dimq_conv2d_lut_full_workspace_bytes(
         dt(xc), B, C, H, W, out_channels, in_channels_per_group, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
         dilation_h, dilation_w, groups, dt(cb)), xc);
-  const On on(xc);
   check_rc(dimq_conv2d_lut_ws(ptr(xc), dt(xc), B, C, H, W, u8(pw), pw.numel(), ptr(cb), dt(cb), cb.numel(), act_scale,
                               act_zp, b.p, b.dtype, b.n, out_channels, in_channels_per_group, kernel_h, kernel_w,
                               stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, groups,
@@ -197,10 +197,10 @@ Tensor linear_codebook(const Tensor& x, const Tensor& packed_w, const Tensor& co
   const Tensor y = at::empty(shape, x.options().dtype(out_dtype.value_or(x.scalar_type())));
   const Residual r(residual, shape, at::MemoryFormat::Contiguous);
   const int nb = static_cast<int>(bits), act = static_cast<int>(activation), var = static_cast<int>(variant);
+  const On on(xc);
   const Tensor ws =
       spare_workspace(dimq_linear_codebook_full_workspace_bytes(M, in_features, out_features, nb, dt(xc)), xc);
   const int64_t wsn = ws.defined() ? ws.numel() : 0;
-  const On on(xc);
   if (!decoded) {
     check_rc(dimq_linear_codebook_ex_ws(ptr(xc), dt(xc), M, in_features, u8(pw), pw.numel(), nb, ptr(cb), dt(cb), rows,
                                         size, b.p, b.dtype, out_features, ptr(y), dt(y), r.p, r.dtype, act, var,
@@ -246,10 +246,10 @@ Tensor conv2d_codebook(const Tensor& x, const Tensor& packed_w, const Tensor& co
   const int64_t prep_words = prep.defined() ? prep.numel() : 0;
   const Residual r(residual, y.sizes(), mf);
   const int nb = static_cast<int>(bits), act = static_cast<int>(activation), var = static_cast<int>(variant);
+  const On on(xc);
   const Tensor ws = spare_workspace(dimq_conv2d_codebook_workspace_bytes(
       dt(xc), layout, B, C, H, W, nb, prep_words > 0, dt(cb), rows, size, out_channels, kernel_h, kernel_w, stride_h,
       stride_w, pad_h, pad_w, dilation_h, dilation_w, groups, dt(y), layout, r.p != nullptr, act, var), xc);
-  const On on(xc);
   check_rc(dimq_conv2d_codebook_ex_ws(ptr(xc), dt(xc), layout, B, C, H, W, u8(pw), pw.numel(), nb,
                                       static_cast<const uint32_t*>(ptr(prep)), prep_words, ptr(cb), dt(cb), rows, size,
                                       b.p, b.dtype, out_channels, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
