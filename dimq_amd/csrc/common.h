@@ -136,6 +136,23 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// s_waitcnt vmcnt(n), leaving the other counters alone (gfx9 encoding:
+// vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]).
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// One global_load_lds of 16 bytes per lane into LDS at byte address lds + 16 * lane.
+// Issued as inline assembly so that the compiler's wait insertion, which
+// would otherwise make every later LDS read wait for all such loads still in
+// flight (it cannot tell the ring's slots apart), leaves the waits to the
+// kernel: wait_vmcnt before the barrier that publishes a stage.
+__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds) {
+  asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
+}
+
 // Load element i of a float tensor of runtime dtype as fp32.
 __device__ __forceinline__ float load_as_float(const void* p, int dt, int64_t i) {
   switch (dt) {

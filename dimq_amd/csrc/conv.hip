@@ -472,9 +472,8 @@ extern "C" int dimq_conv2d_codebook_ex(const void* x, int x_dtype, int x_layout,
 // kernel's own test holds.
 enum ConvPath { kConvGemm, kConvHalo, kConvStem, kConvGeneral };
 
-static ConvPath conv_path(const ConvShape& s, int x_dtype, int x_layout, int y_dtype, int y_layout, int bits,
-                          bool prepared, int mode, int variant, bool x16, bool yw16, bool stem) {
-  (void)y_dtype;
+static ConvPath conv_path(const ConvShape& s, int x_dtype, int x_layout, int y_layout, int bits, bool prepared,
+                          int mode, int variant, bool x16, bool yw16, bool stem) {
   const int64_t hw = prepared ? halo_part_words(s.OC, s.C, s.KH, s.KW, bits) : 0;
   const int64_t gw = prepared ? gemm_part_words(s.OC, s.C, s.KH, s.KW, bits) : 0;
   const bool gemm_ok = gw > 0 && variant != DIMQ_VARIANT_SMALL_M && s.groups == 1 && x_layout == DIMQ_NHWC &&
@@ -514,8 +513,8 @@ extern "C" int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layou
   const bool stem = stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits,
                                   x_dtype, y_dtype, al, al, mode, static_cast<const uint8_t*>(al),
                                   (s.OC * s.ICg * s.KH * s.KW * bits + 7) / 8, al, cb_dtype, cb_rows, cb_size);
-  const ConvPath path = conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared != 0, mode, variant, true,
-                                  true, stem);
+  const ConvPath path = conv_path(s, x_dtype, x_layout, y_layout, bits, prepared != 0, mode, variant, true, true,
+                                  stem);
   if (path == kConvGemm) {
     const int64_t M = B * s.OH * s.OW;
     const int sp = gemm_conv_splits(M, s.OC, s.ICg * s.KH * s.KW);
@@ -568,7 +567,7 @@ extern "C" int dimq_conv2d_codebook_ex_ws(const void* x, int x_dtype, int x_layo
   const bool stem = stem_eligible(s.C, s.OC, s.KH, s.KW, s.sh, s.sw, s.pw, s.dh, s.dw, s.groups, s.OH, s.OW, bits,
                                   x_dtype, y_dtype, x, y, mode, packed_w, packed_numel, codebook, cb_dtype, cb_rows,
                                   cb_size);
-  const ConvPath path = conv_path(s, x_dtype, x_layout, y_dtype, y_layout, bits, prepared_w != nullptr, mode, variant,
+  const ConvPath path = conv_path(s, x_dtype, x_layout, y_layout, bits, prepared_w != nullptr, mode, variant,
                                   aligned(x, 16), aligned(y, 16) && aligned(prepared_w + hw, 16), stem);
   if (path == kConvGemm) {
     GemmArgs p = conv_args(s, x, x_layout, reinterpret_cast<const uint8_t*>(prepared_w + hw), codebook, cb_dtype,

@@ -552,8 +552,8 @@ int64_t stem_rows(int64_t KH, int64_t OH, int64_t OW, int np) {
 // eighths of one round of `slots` work-groups (filled to the last: 64x64 images,
 // batch 64, 20.8 us against 18.9).  A work-group's chain is the weight decode
 // plus a time in proportion to its rows, and a small batch leaves slots idle.
-// ResNet-18 stem, 224x224: batch 1 28.6 -> 16.0 us, 4 29.3 -> 20.6, 8 30.4 ->
-// 24.0, 16 32.1 -> 30.4; from 32 on the bands keep their eight rows.
+// ResNet-18 stem, 224x224: batch 1 28.7 -> 15.4 us, 4 29.7 -> 19.8, 8 30.7 ->
+// 22.8, 16 31.9 -> 29.0; from 32 on the bands keep their eight rows.
 // Bands of whole 8-pixel runs stay so (the NCHW stores' vectors).
 int64_t stem_call_rows(int64_t rows, int64_t B, int64_t OH, int64_t OW, int64_t slots) {
   const bool runs = rows * OW % 8 == 0;

@@ -13,7 +13,7 @@
 //      fp16 channels-last (or row-major) activations whose channel count is
 //      a multiple of 8 are read in place.
 //   2. gen_gemm_kernel: an fp16 GEMM whose operands reach LDS through
-//      global_load_lds in a ring of 32-k stages, as gemm_pd.hip's.  A lane's
+//      global_load_lds in a ring of 64-k stages, after gemm_pd.hip's.  A lane's
 //      16-byte chunk is 8 channels of one tap of one output pixel: its
 //      address is formed per stage from the lane's running (tap, channel),
 //      and chunks outside the image or past the last tap come from a zeroed
@@ -48,18 +48,6 @@ constexpr int64_t kGenActBytes = 256ll << 20;
 // Chunk c of stage row r lies at 128 r + ((c ^ gen_swz(r)) << 4), so that the
 // 16 rows of one 16-byte LDS read cover all 64 banks.
 __device__ __forceinline__ int gen_swz(int r) { return (r >> 1) & (kGenCH - 1); }
-
-template <int N>
-__device__ __forceinline__ void gen_wait_vmcnt() {  // gfx9 s_waitcnt encoding, only vmcnt
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// 16 bytes per lane into LDS at lds + 16 * lane; inline assembly so that the
-// compiler's wait insertion leaves the ring's waits to the kernel.
-__device__ __forceinline__ void gen_dma16(const void* gptr, uint32_t lds) {
-  asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
 
 struct GenArgs {
   // first launch
@@ -188,7 +176,7 @@ __device__ void gen_weight_rows(const GemmArgs& p, const GenArgs& a, int64_t b) 
   }
 }
 
-// 8 activations (the last `n` of them real) -> fp16 or W4A4 codes.
+// 8 activations (the first `n` of them real) -> fp16 or W4A4 codes.
 __device__ __forceinline__ uint4 gen_convert8(const GemmArgs& p, const GenArgs& a, float (&v)[8], int n) {
   if (a.a4) u4_codes<8>(v, p.act_scale, p.act_zp);
 #pragma unroll
@@ -455,7 +443,7 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const GemmArgs p, const G
     const uint32_t dst = smb + slot * RSTAGE + wave * 1024;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      gen_dma16(wsrc[j], dst + j * NW * 1024);
+      dma16(wsrc[j], dst + j * NW * 1024);
       wsrc[j] += kGenK;
     }
     if constexpr (CONV) {
@@ -467,7 +455,7 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const GemmArgs p, const G
         const bool in = tap_in && static_cast<uint32_t>(ih0[j] + dh) < static_cast<uint32_t>(p.cH) &&
                         static_cast<uint32_t>(iw0[j] + dw) < static_cast<uint32_t>(p.cW);
         const void* src = in ? static_cast<const void*>(xg + (xoff[j] + delta)) : static_cast<const void*>(a.zero);
-        gen_dma16(src, dst + (J + j) * NW * 1024);
+        dma16(src, dst + (J + j) * NW * 1024);
       }
       if (++ka == nka) {  // the second weight plane starts over
         ka = 0;
@@ -482,7 +470,7 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const GemmArgs p, const G
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < J; ++j) gen_dma16(xsrc[j] + ka * kGenK, dst + (J + j) * NW * 1024);
+      for (int j = 0; j < J; ++j) dma16(xsrc[j] + ka * kGenK, dst + (J + j) * NW * 1024);
       if (++ka == nka) ka = 0;
     }
   };
@@ -518,16 +506,16 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const GemmArgs p, const G
   const int64_t nk = k1 - k0;
 #pragma unroll
   for (int s = 0; s < S; ++s) issue(k0 + s, s);
-  if (nk >= S) gen_wait_vmcnt<(S - 1) * LPS>();
-  else gen_wait_vmcnt<0>();
+  if (nk >= S) wait_vmcnt<(S - 1) * LPS>();
+  else wait_vmcnt<0>();
   lds_barrier();
   load(0, std::integral_constant<int, 0>());
   int slot = 0;
   auto step = [&](int64_t kt, auto curc) {  // kt + 1 < nk
     constexpr int CUR = decltype(curc)::value;
     const int next = slot == S - 1 ? 0 : slot + 1;
-    if (kt + S <= nk) gen_wait_vmcnt<(S - 2) * LPS>();  // stages kt + 2 .. kt + S - 1 may be in flight
-    else gen_wait_vmcnt<0>();
+    if (kt + S <= nk) wait_vmcnt<(S - 2) * LPS>();  // stages kt + 2 .. kt + S - 1 may be in flight
+    else wait_vmcnt<0>();
     lds_barrier();
     issue(k0 + kt + S, slot);
     load(next, std::integral_constant<int, 1 - CUR>());

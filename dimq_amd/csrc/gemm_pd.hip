@@ -46,23 +46,6 @@ __device__ __forceinline__ int pd_swz(int r) {
   return (r / (16 / CH)) & (CH - 1);
 }
 
-// s_waitcnt vmcnt(n), leaving the other counters alone (gfx9 encoding:
-// vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// One global_load_lds of 16 bytes per lane into LDS at byte address lds + 16 * lane.
-// Issued as inline assembly so that the compiler's wait insertion, which
-// would otherwise make every later LDS read wait for all such loads still in
-// flight (it cannot tell the ring's slots apart), leaves the waits to the
-// kernel: wait_vmcnt before the barrier that publishes a stage.
-__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds) {
-  asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
-
 constexpr int kPdRows = 4;     // weight rows per predecode work-group (2: 10.1 us, 4: 9.3, 8: slower, per ViT-B/16 block)
 constexpr int kPdGroups = 16;  // 8-index groups per thread held in registers (K <= 4096 in one pass)
 
