@@ -521,6 +521,13 @@ extern "C" int64_t dimq_conv2d_codebook_workspace_bytes(int x_dtype, int x_layou
     return sp > 1 ? split_bytes(sp, M, s.OC) : 0;
   }
   if (path != kConvGeneral) return 0;
+  // No cost rule: every shape tried that the others leave is faster here than on
+  // gemm_cb_kernel's im2col tiles, groups of few channels too, although each is
+  // padded to 8 channels and a tile of 64 columns (fp16, channels last: depthwise
+  // 3x3, 8 x 512 x 14 x 14 365 -> 158 us; stride 2, 32 x 96 x 56 x 56 1,099 ->
+  // 808; 32 groups of 4 channels, 8 x 128 x 56 x 56 528 -> 145; of 32, 8 x 1,024
+  // x 7 x 7 47 -> 10), single outputs (1x1, 8 x 64 x 56 x 56 to one channel 26 ->
+  // 10) and single pixels (1 x 2,048 to 1,000 78 -> 15).
   const GenPlan g = gen_plan(shape_args(s, x_layout, y_layout, DIMQ_F32), bits, x_dtype, false, true);
   return g.ok ? g.bytes : 0;
 }
