@@ -745,7 +745,10 @@ GenPlan gen_plan(const GemmArgs& p, int bits, int x_dtype, bool a4, bool in_plac
   if (units * unit_bytes > kGenActBytes) {
     const int64_t most = unit_bytes < kGenActBytes ? kGenActBytes / unit_bytes : 1;
     g.step = cdiv(units, cdiv(units, most));  // passes of about the same size
-    if (!g.conv && most >= kGenB) g.step = cdiv(g.step, kGenB) * kGenB <= most ? cdiv(g.step, kGenB) * kGenB : most / kGenB * kGenB;
+    if (!g.conv && most >= kGenB) {  // whole tiles of rows
+      const int64_t up = cdiv(g.step, kGenB) * kGenB;
+      g.step = up <= most ? up : most / kGenB * kGenB;
+    }
     g.pixels = g.pixels / units * g.step;
   }
   const int64_t M = p.M / units * g.step;  // rows of a pass

@@ -16,11 +16,12 @@
 // and the softmin term is dmin_i - tau log(s_i / K).  For s_i > K / 2
 // (near-uniform p: large tau) log(s_i / K) is formed as
 // log1p(sum_j expm1(-(d_ij - dmin_i) / tau) / K), since log s_i - log K would
-// cancel to a few digits there; otherwise as log s_i - log K.  The forward kernels store
-// (dmin_i, 1 / s_i) per element, so a backward pass gets p_ij without a second
-// pass over the centres (and with no rounding of a logarithm in its exponent).
-// Sums over elements (the loss, the centre gradients) go through per-work-group partials and a final pass in a fixed order:
-// results do not depend on scheduling.
+// cancel to a few digits there; otherwise as log s_i - log K.  The forward
+// kernels store (dmin_i, 1 / s_i) per element, so a backward pass gets p_ij
+// without a second pass over the centres (and with no rounding of a logarithm in
+// its exponent).  Sums over elements (the loss, the centre gradients) go through
+// per-work-group partials and a final pass in a fixed order: results do not
+// depend on scheduling.
 #include <type_traits>
 
 #include "common.h"
